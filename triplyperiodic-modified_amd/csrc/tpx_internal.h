@@ -220,6 +220,16 @@ struct TileTune {
   std::vector<Pending> pending;
 };
 
+// Pinned chunks that downloads pass through, and the events of the copies in
+// flight: two per copying thread, made on the first download that uses them.
+constexpr size_t kStageChunk = 1u << 20;
+constexpr int kStageMaxThreads = 4;
+struct HostStage {
+  char *pin[kStageMaxThreads] = {};
+  hipEvent_t ev[kStageMaxThreads][2] = {};
+  int threads = 0;
+};
+
 struct Timing {
   bool on = false;
   struct Rec { int cls; hipEvent_t a, b; };
@@ -297,6 +307,7 @@ struct tpx_ctx {
   int32_t *scan_tmp = nullptr;    // scan block sums
   tpx::Particles pt;
   tpx::Timing tm;
+  tpx::HostStage stage;
   std::string err;
 };
 

@@ -194,9 +194,7 @@ class Solver:
         if name in VECTOR:
             out = np.empty((3,) + sh)
             for c in range(3):
-                a = np.empty(sh)
-                self._ok(self.L.tpx_download_field(self.h, fid, c, _dp(a), bs), f"download {name}")
-                out[c] = a
+                self._ok(self.L.tpx_download_field(self.h, fid, c, _dp(out[c]), bs), f"download {name}")
             return out
         out = np.empty(sh)
         self._ok(self.L.tpx_download_field(self.h, fid, 0, _dp(out), bs), f"download {name}")
