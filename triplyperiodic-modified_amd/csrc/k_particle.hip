@@ -943,7 +943,17 @@ void launch_particle_advance(tpx_ctx *c, const Coef &k, const double *const ru_i
 // Launch shape of the heat moment and velocity deposit kernels: `rows` whole
 // x-rows per block and `zc` planes per z-march.  The built-in choice is 256
 // threads (nx when nx > 256) and up to 32 planes (8 for the velocity
-// deposit); a tuned or set shape replaces it.
+// deposit); a tuned or set shape replaces it.  A march is a serial chain of
+// planes, so a small grid takes shorter ones until the launch (over every box
+// of a batch) fills the chip: the heat march, which re-does two halo planes
+// per block, down to 2 planes below 2^17 threads (two blocks a CU), the
+// velocity march, whose halo is one plane of one share, down to 1 below 2^20.
+// Below 256 blocks the heat march then takes fewer rows, down to one wave, and
+// single planes.  Both deposits together, heat shape changed alone: 32^3 139
+// -> 38 us, 64^3 131 -> 43, 128 x 32 x 64 143 -> 46, 128^3 162 -> 123, while
+// 512 x 64 x 128 and 256^3 are fastest at 32 planes (213 against 217 and 898
+// against 913 us at 16); velocity shape alone: 64^3 134 -> 122, 128 x 32 x 64
+// 144 -> 132, 128^3 168 -> 163, 512 x 64 x 128 217 -> 210.
 struct HeatShape { int threads, rows, zc; unsigned blocks; };
 static HeatShape deposit_shape(const tpx_ctx *c, int kind) {
   const Geo &g = c->g;
@@ -951,6 +961,17 @@ static HeatShape deposit_shape(const tpx_ctx *c, int kind) {
   HeatShape h;
   h.rows = set.rows > 0 ? set.rows : (g.nx >= 256 ? 1 : std::min(256 / g.nx, g.ny));
   h.zc = set.zc > 0 ? set.zc : std::min(kind == 0 ? 32 : 8, g.nz);
+  const long nbox = g_rec ? g_rec->nbox : 1;
+  auto blocks = [&]() { return nbox * (g.ny / h.rows) * (g.nz / h.zc); };
+  if (set.rows <= 0 && set.zc <= 0) {
+    const int zmin = kind == 0 ? 2 : 1;
+    const long fill = kind == 0 ? 1L << 17 : 1L << 20;
+    while (h.zc > zmin && blocks() * g.nx * h.rows < fill) h.zc /= 2;
+    if (kind == 0) {
+      while (h.rows > 1 && g.nx * h.rows > 64 && blocks() < 256) h.rows /= 2;
+      if (blocks() < 256) h.zc = 1;
+    }
+  }
   h.threads = g.nx * h.rows;
   h.blocks = (unsigned)((g.ny / h.rows) * (g.nz / h.zc));
   return h;
