@@ -154,6 +154,8 @@ struct XArgs {
                          // caller's face coefficient), or null: formed here from rho
   const double *in = nullptr;  // three-pass form: transform this field's rows instead of a
                                // residual (P, rho, rhs unread)
+  const double *cf[3] = {};    // three-pass form, its own kernel instance: the caller's face
+                               // coefficient in the place of 1 / Rho_face (rho unread, RHS as given)
   __device__ void to_global() {
     P = gptr(P);
     rho = gptr(rho);
@@ -164,6 +166,7 @@ struct XArgs {
     done = gptr(done);
     res = gptr(res);
     in = gptr(in);
+    for (auto &q : cf) q = gptr(q);
   }
 };
 
@@ -275,6 +278,18 @@ __device__ __forceinline__ void row_residuals(const XArgs &a, const Ix &ix, int 
     rcur = rn;
     cx0 = cx0n;
   }
+}
+
+// the residual at cell (i,j,k) with the caller's face coefficient and RHS as
+// given (poisson.cpp:391-411); C.x at the low x face of its cell
+__device__ __forceinline__ double residual_coef(const XArgs &a, const Ix &ix, int i, int j, int k) {
+  const double *__restrict__ P = a.P;
+  const double *__restrict__ cx = a.cf[0];
+  const double *__restrict__ cy = a.cf[1];
+  const double *__restrict__ cz = a.cf[2];
+  const long e = ix(i, j, k), xp = ix(i + 1, j, k), yp = ix(i, j + 1, k), zp = ix(i, j, k + 1);
+  return residual_of(a.g, P[e], P[ix(i - 1, j, k)], P[xp], P[ix(i, j - 1, k)], P[yp], P[ix(i, j, k - 1)], P[zp], cx[e],
+                     cx[xp], cy[e], cy[yp], cz[e], cz[zp], a.rhs[e], 0.0);
 }
 
 // X forward pass: lpb consecutive x lines per block
@@ -867,7 +882,7 @@ struct k_zpass4 {
 // the five-pass form.
 constexpr int kRunPad = 8;  // spare complex values after each nz Y1 run
 // ---------------------------------------------------------------------------
-template <int R1, int R2, int Y2>
+template <int R1, int R2, int Y2, bool Coef = false>
 struct k_xy_fwd {
   static constexpr int kBounds = 256;
   static __device__ __forceinline__ void run(const XArgs &a, int Y1, const double2 *__restrict__ twy) {
@@ -885,7 +900,10 @@ struct k_xy_fwd {
   double2 v[R2];
   {
     const int j = t + Y1 * ca;
-    if (a.in) {
+    if constexpr (Coef) {
+#pragma unroll
+      for (int m = 0; m < R2; ++m) v[m] = make_double2(residual_coef(a, ix, ta + R1 * m, j, z), 0.0);
+    } else if (a.in) {
       const double *row = a.in + (long)z * g.nxy + (long)j * g.nx + ta;
 #pragma unroll
       for (int m = 0; m < R2; ++m) v[m] = make_double2(row[R1 * m], 0.0);
@@ -1177,9 +1195,52 @@ __device__ __forceinline__ void row_residuals_pairs(const XArgs &a, const Ix &ix
   }
 }
 
+// the same pairs with the caller's face coefficient: 11 loads of 16 bytes a
+// pair, the x neighbours from the lanes beside it
+template <int R2H>
+__device__ __forceinline__ void row_residuals_pairs_coef(const XArgs &a, const Ix &ix, int ta, int j, int z,
+                                                         double2 (&v)[R2H]) {
+  const double *__restrict__ P = a.P;
+  const double *__restrict__ cx = a.cf[0];
+  const double *__restrict__ cy = a.cf[1];
+  const double *__restrict__ cz = a.cf[2];
+  const double *__restrict__ rhs = a.rhs;
+  const long zc = (long)(z & ix.mz) * ix.nxy, yc = (long)(j & ix.my) * ix.nx;
+  const long rc = zc + yc, ryl = zc + (long)((j - 1) & ix.my) * ix.nx, ryh = zc + (long)((j + 1) & ix.my) * ix.nx;
+  const long rzl = (long)((z - 1) & ix.mz) * ix.nxy + yc, rzh = (long)((z + 1) & ix.mz) * ix.nxy + yc;
+  auto ld2 = [&](const double *f, long row, int m) {
+    return *reinterpret_cast<const double2 *>(f + row + 2 * ta + 32 * m);
+  };
+  auto lo_of = [&](double cur_odd, double prev_odd) {
+    const double u = row_rotate<0x121>(cur_odd), w = row_rotate<0x121>(prev_odd);
+    return ta == 0 ? w : u;
+  };
+  auto hi_of = [&](double cur_even, double next_even) {
+    const double u = row_rotate<0x12F>(cur_even), w = row_rotate<0x12F>(next_even);
+    return ta == 15 ? w : u;
+  };
+  double2 pp = ld2(P, rc, R2H - 1), pc = ld2(P, rc, 0), xc = ld2(cx, rc, 0);
+#pragma unroll
+  for (int m = 0; m < R2H; ++m) {
+    const int mn = (m + 1) % R2H;
+    const double2 pn = ld2(P, rc, mn), xn = ld2(cx, rc, mn);
+    const double2 pym = ld2(P, ryl, m), pyp = ld2(P, ryh, m), pzm = ld2(P, rzl, m), pzp = ld2(P, rzh, m);
+    const double2 y0 = ld2(cy, rc, m), y1 = ld2(cy, ryh, m), z0 = ld2(cz, rc, m), z1 = ld2(cz, rzh, m);
+    const double2 r0 = ld2(rhs, rc, m);
+    const double ra = residual_of(a.g, pc.x, lo_of(pc.y, pp.y), pc.y, pym.x, pyp.x, pzm.x, pzp.x, xc.x, xc.y, y0.x,
+                                  y1.x, z0.x, z1.x, r0.x, 0.0);
+    const double rb = residual_of(a.g, pc.y, pc.x, hi_of(pc.x, pn.x), pym.y, pyp.y, pzm.y, pzp.y, xc.y,
+                                  hi_of(xc.x, xn.x), y0.y, y1.y, z0.y, z1.y, r0.y, 0.0);
+    v[m] = make_double2(ra, rb);
+    pp = pc;
+    pc = pn;
+    xc = xn;
+  }
+}
+
 // pass 1, packed: residual rows, the M-point x transform, the half spectrum
 // recovered on the way out of LDS, y step A
-template <int R2H, int Y2>
+template <int R2H, int Y2, bool Coef = false>
 struct k_xy_fwd_rp {
   static constexpr int kBounds = 256;
   static __device__ __forceinline__ void run(const XArgs &a, int Y1, const double2 *__restrict__ twy) {
@@ -1194,7 +1255,9 @@ struct k_xy_fwd_rp {
     const int t = (int)(blk % (unsigned)Y1), z = (int)(blk / (unsigned)Y1);
     const int ta = threadIdx.x % R1, ca = threadIdx.x / R1;
     double2 v[R2H];
-    if (a.in) {
+    if constexpr (Coef) {
+      row_residuals_pairs_coef<R2H>(a, ix, ta, t + Y1 * ca, z, v);
+    } else if (a.in) {
       const double *row = a.in + (long)z * g.nxy + (long)(t + Y1 * ca) * g.nx + 2 * ta;
 #pragma unroll
       for (int m = 0; m < R2H; ++m) v[m] = *reinterpret_cast<const double2 *>(row + 32 * m);
@@ -1489,22 +1552,32 @@ static bool four_step(int n, int &r1, int &r2) {
 
 // launch helpers of the three-pass iteration: template arguments from the
 // run-time factorisations
-template <int R1, int R2>
-void xy_fwd_launch(unsigned nb, size_t sh, hipStream_t st, const XArgs &xa, int Y1, int Y2, const double2 *twy) {
+template <int R1, int R2, bool Coef>
+void xy_fwd_launch_t(unsigned nb, size_t sh, hipStream_t st, const XArgs &xa, int Y1, int Y2, const double2 *twy) {
   switch (Y2) {
-    case 4: tpx_launch<k_xy_fwd<R1, R2, 4>>(nb, 4 * R1, sh, st, xa, Y1, twy); break;
-    case 8: tpx_launch<k_xy_fwd<R1, R2, 8>>(nb, 8 * R1, sh, st, xa, Y1, twy); break;
-    default: tpx_launch<k_xy_fwd<R1, R2, 16>>(nb, 16 * R1, sh, st, xa, Y1, twy); break;
+    case 4: tpx_launch<k_xy_fwd<R1, R2, 4, Coef>>(nb, 4 * R1, sh, st, xa, Y1, twy); break;
+    case 8: tpx_launch<k_xy_fwd<R1, R2, 8, Coef>>(nb, 8 * R1, sh, st, xa, Y1, twy); break;
+    default: tpx_launch<k_xy_fwd<R1, R2, 16, Coef>>(nb, 16 * R1, sh, st, xa, Y1, twy); break;
   }
 }
+template <int R1, int R2>
+void xy_fwd_launch(unsigned nb, size_t sh, hipStream_t st, const XArgs &xa, int Y1, int Y2, const double2 *twy) {
+  if (xa.cf[0]) xy_fwd_launch_t<R1, R2, true>(nb, sh, st, xa, Y1, Y2, twy);
+  else xy_fwd_launch_t<R1, R2, false>(nb, sh, st, xa, Y1, Y2, twy);
+}
 // the packed forward form for x lengths 64, 128 and 256 (R2H = 2, 4, 8)
+template <int R2H, bool Coef>
+void xy_fwd_rp_launch_t(unsigned nb, size_t sh, hipStream_t st, const XArgs &xa, int Y1, int Y2, const double2 *twy) {
+  switch (Y2) {
+    case 4: tpx_launch<k_xy_fwd_rp<R2H, 4, Coef>>(nb, 4 * 16, sh, st, xa, Y1, twy); break;
+    case 8: tpx_launch<k_xy_fwd_rp<R2H, 8, Coef>>(nb, 8 * 16, sh, st, xa, Y1, twy); break;
+    default: tpx_launch<k_xy_fwd_rp<R2H, 16, Coef>>(nb, 16 * 16, sh, st, xa, Y1, twy); break;
+  }
+}
 template <int R2H>
 void xy_fwd_rp_launch(unsigned nb, size_t sh, hipStream_t st, const XArgs &xa, int Y1, int Y2, const double2 *twy) {
-  switch (Y2) {
-    case 4: tpx_launch<k_xy_fwd_rp<R2H, 4>>(nb, 4 * 16, sh, st, xa, Y1, twy); break;
-    case 8: tpx_launch<k_xy_fwd_rp<R2H, 8>>(nb, 8 * 16, sh, st, xa, Y1, twy); break;
-    default: tpx_launch<k_xy_fwd_rp<R2H, 16>>(nb, 16 * 16, sh, st, xa, Y1, twy); break;
-  }
+  if (xa.cf[0]) xy_fwd_rp_launch_t<R2H, true>(nb, sh, st, xa, Y1, Y2, twy);
+  else xy_fwd_rp_launch_t<R2H, false>(nb, sh, st, xa, Y1, Y2, twy);
 }
 template <int R1, int R2, bool Ow, bool Oop>
 void xy_inv_launch_t(unsigned nb, size_t sh, hipStream_t st, const XInvArgs &xi, int Y1, int Y2, const double2 *twy) {
@@ -1577,7 +1650,11 @@ unsigned three_pass_launch(tpx_ctx *c, const XArgs &xa, const XInvArgs &xi, cons
   // the full-length inverse (the same half spectrum either way: the packed
   // inverse, whose final stage leaves half the block idle over the P
   // update, measured slower)
-  const bool packed = (g.nx == 64 || g.nx == 128 || g.nx == 256) && c->x_packed;
+  // the packed form reads pairs with 16-byte loads: the library's own fields
+  // are aligned, a caller's arrays (coefficient solve) need not be
+  bool packed = (g.nx == 64 || g.nx == 128 || g.nx == 256) && c->x_packed;
+  if (xa.cf[0])
+    for (const double *q : {xa.cf[0], xa.cf[1], xa.cf[2], xa.P, xa.rhs}) packed = packed && (uintptr_t)q % 16 == 0;
 #define L_XYF(A, B) xy_fwd_launch<A, B>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1])
   if (packed && g.nx == 256) xy_fwd_rp_launch<8>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1]);
   else if (packed && g.nx == 128) xy_fwd_rp_launch<4>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1]);
@@ -1699,6 +1776,31 @@ void launch_poisson_iteration_on(tpx_ctx *c, const double *rho_new, double *P, c
   tpx_launch<k_finish_iter>(1, 1024, 0, c->stream, c->partials, nbx, scal, c->Iteration, c->p.epsilon);
   TPX_LAUNCH_CHECK();
   timing_end(c, TPX_K_FFT_INV);
+}
+
+// One iteration with the caller's face coefficient: pass 1 of the three-pass
+// form reads it in the place of 1 / Rho_face; where an axis rules that form
+// out, the residual is formed into `res` and goes through the five passes.
+// (Every size took the residual kernel and the five passes before, seven
+// launches and two more passes over the residual: whole solves 558 -> 401 us
+// at 32^3 (12 iterations), 1299 -> 906 us at 128^3 (13).)
+void launch_coef_iteration(tpx_ctx *c, const double *const cf[3], double *P, const double *rhs, double *res) {
+  const Geo &g = c->g;
+  int r1, r2, y1, y2, z1, z2;
+  if (three_pass_shape(c, r1, r2, y1, y2, z1, z2)) {
+    const double *done = c->scal + SC_DONE;
+    timing_begin(c, TPX_K_FFT);
+    XArgs xa{g, P, nullptr, rhs, c->scal, c->spec[0], c->tw[0], (double)g.n, done, nullptr};
+    for (int d = 0; d < 3; ++d) xa.cf[d] = cf[d];
+    const XInvArgs xi{g, P, c->spec[0], c->tw[0], c->partials, (double)g.n, done};
+    const unsigned nb13 = three_pass_launch(c, xa, xi, done, r1, r2, y1, y2);
+    tpx_launch<k_finish_iter>(1, 1024, 0, c->stream, c->partials, nb13, c->scal, c->Iteration, c->p.epsilon);
+    TPX_LAUNCH_CHECK();
+    timing_end(c, TPX_K_FFT_INV);
+    return;
+  }
+  launch_residual_coef(c, cf, P, rhs, res);
+  launch_poisson_iteration_on(c, nullptr, P, rhs, c->scal, res);
 }
 
 void launch_spectral_apply(tpx_ctx *c, const double *in, double *out, double *scal) {

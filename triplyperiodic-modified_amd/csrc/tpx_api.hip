@@ -438,14 +438,10 @@ void do_solve_poisson(tpx_ctx *c, int rk, int *iters, const std::function<void(i
   if (iters) *iters = i;
 }
 
-// poisson::FFT with the caller's face coefficient (poisson.cpp:391-411): each
-// iteration forms the residual in its own kernel into `res` and runs the
-// five-pass transform on it.  P, RHS, C and res are dense device arrays.
+// poisson::FFT with the caller's face coefficient (poisson.cpp:391-411).  P,
+// RHS, C and res (work) are dense device arrays.
 void do_solve_coef(tpx_ctx *c, const double *const cf[3], double *P, const double *rhs, double *res, int *iters) {
-  const int i = solve_loop(c, 2, [&](int) {
-    launch_residual_coef(c, cf, P, rhs, res);
-    launch_poisson_iteration_on(c, nullptr, P, rhs, c->scal, res);
-  });
+  const int i = solve_loop(c, 2, [&](int) { launch_coef_iteration(c, cf, P, rhs, res); });
   c->num_iteration = i;  // the reference's poisson object keeps the last solve's count
   if (iters) *iters = i;
 }

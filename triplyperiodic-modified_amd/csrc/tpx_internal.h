@@ -353,6 +353,8 @@ void launch_poisson_iteration_on(tpx_ctx *c, const double *rho_new, double *P, c
 // division by the modified wavenumbers, inverse, -1/ncell): the iteration's
 // dp for the residual `in`.  No loop test runs; scal[SC_DONE] must be 0.
 void launch_spectral_apply(tpx_ctx *c, const double *in, double *out, double *scal);
+// one iteration with a caller's face coefficient C (cf[0..2]); res: work of n values
+void launch_coef_iteration(tpx_ctx *c, const double *const cf[3], double *P, const double *rhs, double *res);
 // r = (div_F2C(C grad_C2F P) - RHS) cc for a caller's face coefficient C (cf[0..2])
 void launch_residual_coef(tpx_ctx *c, const double *const cf[3], const double *P, const double *rhs, double *res);
 // the passive vector (k_vector.hip): Update_RV_WOQ, Compute_RHS_Pois_Q (raw
