@@ -149,7 +149,8 @@ struct XArgs {
   double2 *spec;
   const double2 *tw;     // x twiddles
   double ncell;
-  const double *done;    // nonzero: the solve has converged, the iteration is skipped
+  const double *done;    // nonzero: the solve has converged, the iteration is skipped (null: the
+                         // solve's first iteration, which always runs)
   const double *res;     // the residual formed by k_residual_coef (a solve with the
                          // caller's face coefficient), or null: formed here from rho
   const double *in = nullptr;  // three-pass form: transform this field's rows instead of a
@@ -296,7 +297,7 @@ __device__ __forceinline__ double residual_coef(const XArgs &a, const Ix &ix, in
 struct k_xfwd {
   static constexpr int kBounds = kThreads;
   static __device__ __forceinline__ void run(const XArgs &a, int lpb) {
-  if (*a.done != 0.0) return;  // the solve has converged
+  if (a.done && *a.done != 0.0) return;  // the solve has converged
   extern __shared__ double2 lds[];
   const Geo &g = a.g;
   int nx = g.nx, mxh = nx / 2 + 1;
@@ -346,7 +347,7 @@ struct XInvArgs {
 struct k_xinv {
   static constexpr int kBounds = kThreads;
   static __device__ __forceinline__ void run(const XInvArgs &a, int lpb) {
-  if (*a.done != 0.0) return;  // the solve has converged
+  if (a.done && *a.done != 0.0) return;  // the solve has converged
   extern __shared__ double2 lds[];
   __shared__ double red[kThreads];
   const Geo &g = a.g;
@@ -391,7 +392,7 @@ struct k_ypass {
   static constexpr int kBounds = kThreads;
   static __device__ __forceinline__ void run(double2 *spec, int mxh, int ny, int nz,
                                                     const double2 *__restrict__ tw, int kTile, const double *__restrict__ done) {
-  if (*done != 0.0) return;  // the solve has converged
+  if (done && *done != 0.0) return;  // the solve has converged
   extern __shared__ double2 lds[];
   int ntile = (mxh + kTile - 1) / kTile;
   unsigned blk = xcd_block(blockIdx.x, gridDim.x);
@@ -421,7 +422,7 @@ struct k_zpass {
                                                     const double *__restrict__ lamx,
                                                     const double *__restrict__ lamy,
                                                     const double *__restrict__ lamz, int kTile, const double *__restrict__ done) {
-  if (*done != 0.0) return;  // the solve has converged
+  if (done && *done != 0.0) return;  // the solve has converged
   extern __shared__ double2 lds[];
   int ntile = (mxh + kTile - 1) / kTile;
   unsigned blk = xcd_block(blockIdx.x, gridDim.x);
@@ -617,7 +618,7 @@ template <int R1, int R2>
 struct k_xfwd4 {
   static constexpr int kBounds = 256;
   static __device__ __forceinline__ void run(const XArgs &a, int C) {
-  if (*a.done != 0.0) return;  // the solve has converged
+  if (a.done && *a.done != 0.0) return;  // the solve has converged
   // The exchange moves real and imaginary parts in two rounds through an
   // LDS buffer of doubles: half the LDS per block, more blocks per CU.
   extern __shared__ double ldsd[];
@@ -674,7 +675,7 @@ template <int R1, int R2>
 struct k_xinv4 {
   static constexpr int kBounds = 256;
   static __device__ __forceinline__ void run(const XInvArgs &a, int C) {
-  if (*a.done != 0.0) return;  // the solve has converged
+  if (a.done && *a.done != 0.0) return;  // the solve has converged
   extern __shared__ double2 lds[];
   __shared__ double red[256];
   constexpr int n = R1 * R2, P = R1 + 1;
@@ -756,7 +757,7 @@ struct k_ypass4 {
   static __device__ __forceinline__ void run(double2 *spec, int mxh, int ny, int nz,
                                                 const double2 *__restrict__ tw, int C,
                                                 const double *__restrict__ done) {
-  if (*done != 0.0) return;  // the solve has converged
+  if (done && *done != 0.0) return;  // the solve has converged
   extern __shared__ double2 lds[];
   const int ntile = (mxh + C - 1) / C;
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
@@ -793,7 +794,7 @@ struct k_zpass4 {
                                                 const double *__restrict__ lamy,
                                                 const double *__restrict__ lamz, int C,
                                                 const double *__restrict__ done) {
-  if (*done != 0.0) return;  // the solve has converged
+  if (done && *done != 0.0) return;  // the solve has converged
   extern __shared__ double2 lds[];
   const int ntile = (mxh + C - 1) / C;
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
@@ -886,7 +887,7 @@ template <int R1, int R2, int Y2, bool Coef = false>
 struct k_xy_fwd {
   static constexpr int kBounds = 256;
   static __device__ __forceinline__ void run(const XArgs &a, int Y1, const double2 *__restrict__ twy) {
-  if (*a.done != 0.0) return;  // the solve has converged
+  if (a.done && *a.done != 0.0) return;  // the solve has converged
   extern __shared__ double ldsd[];
   constexpr int n = R1 * R2, P = R1 + 1, SP = Y2 + 1;  // padded rows of the x exchange and of the kx columns
   const Geo &g = a.g;
@@ -971,7 +972,7 @@ struct k_yz_pass {
                                                  const double *__restrict__ lamy,
                                                  const double *__restrict__ lamz,
                                                  const double *__restrict__ done) {
-  if (*done != 0.0) return;  // the solve has converged
+  if (done && *done != 0.0) return;  // the solve has converged
   extern __shared__ double2 L[];
   constexpr int nz = Z1 * Z2, NE = nz * Y1, RS = nz + nz / 16;
   auto pad = [](int e) { return e + (e >> 4); };  // one spare slot every 16: fewer bank conflicts
@@ -1244,7 +1245,7 @@ template <int R2H, int Y2, bool Coef = false>
 struct k_xy_fwd_rp {
   static constexpr int kBounds = 256;
   static __device__ __forceinline__ void run(const XArgs &a, int Y1, const double2 *__restrict__ twy) {
-    if (*a.done != 0.0) return;  // the solve has converged
+    if (a.done && *a.done != 0.0) return;  // the solve has converged
     extern __shared__ double ldsd[];
     constexpr int R1 = 16, M = R1 * R2H, P = R1 + 1, SP = Y2 + 1;
     const Geo &g = a.g;
@@ -1320,7 +1321,7 @@ template <int R1, int R2, int Y2, bool Overwrite = false, bool OutOfPlace = fals
 struct k_xy_inv {
   static constexpr int kBounds = 256;
   static __device__ __forceinline__ void run(const XInvArgs &a, int Y1, const double2 *__restrict__ twy) {
-  if (*a.done != 0.0) return;  // the solve has converged
+  if (a.done && *a.done != 0.0) return;  // the solve has converged
   extern __shared__ double ldsd[];
   __shared__ double red[256];
   constexpr int n = R1 * R2, P = R1 + 1, SP = Y2 + 1;
@@ -1432,7 +1433,7 @@ struct k_residual_coef {
                                              const double *__restrict__ cz, const double *__restrict__ P,
                                              const double *__restrict__ rhs, double *__restrict__ res,
                                              const double *done) {
-    if (*done != 0.0) return;
+    if (done && *done != 0.0) return;
     const long e = (long)blockIdx.x * block_dim_x() + threadIdx.x;
     if (e >= g.n) return;
     const int i = (int)(e % g.nx), j = (int)((e / g.nx) % g.ny), k = (int)(e / g.nxy);
@@ -1446,9 +1447,9 @@ struct k_residual_coef {
 struct k_finish_iter {
   static constexpr int kBounds = 1024;
   static __device__ __forceinline__ void run(const double *__restrict__ partials, long nparts,
-                                                      double *scal, int iteration, double epsilon) {
+                                                      double *scal, int iteration, double epsilon, const IterCtl &ctl) {
   __shared__ double sh[1024];
-  if (scal[SC_DONE] != 0.0) return;
+  if (!ctl.first && scal[SC_DONE] != 0.0) return;
   double v = 0.0;
   for (long q = threadIdx.x; q < nparts; q += 1024) v = fmax(v, partials[q]);  // coalesced
   sh[threadIdx.x] = v;
@@ -1458,10 +1459,14 @@ struct k_finish_iter {
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    const double err = sh[0], it = scal[SC_ITERS] + 1.0;
+    const double err = sh[0], it = ctl.first ? 1.0 : scal[SC_ITERS] + 1.0;
+    const bool more = it < iteration && err > epsilon;
     scal[SC_MAX_DP] = err;
     scal[SC_ITERS] = it;
-    scal[SC_DONE] = (it < iteration && err > epsilon) ? 0.0 : 1.0;
+    scal[SC_DONE] = more ? 0.0 : 1.0;
+    if (ctl.host)  // the host reads the loop state from its own memory as the solve goes
+      __hip_atomic_store(ctl.host, ((uint64_t)ctl.epoch << 32) | ((uint64_t)it << 1) | (more ? 0 : 1),
+                         __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 };
@@ -1626,7 +1631,7 @@ void launch_poisson_iteration(tpx_ctx *c, const double *rho_new) {
 void launch_residual_coef(tpx_ctx *c, const double *const cf[3], const double *P, const double *rhs, double *res) {
   const Geo &g = c->g;
   tpx_launch<k_residual_coef>((unsigned)((g.n + kThreads - 1) / kThreads), kThreads, 0, c->stream, g, cf[0], cf[1],
-                              cf[2], P, rhs, res, (const double *)(c->scal + SC_DONE));
+                              cf[2], P, rhs, res, c->iter_ctl.first ? nullptr : (const double *)(c->scal + SC_DONE));
   TPX_LAUNCH_CHECK();
 }
 
@@ -1686,7 +1691,7 @@ void launch_poisson_iteration_on(tpx_ctx *c, const double *rho_new, double *P, c
   long nlines = (long)g.ny * g.nz;
   int r1, r2;
   timing_begin(c, TPX_K_FFT);
-  const double *done = scal + SC_DONE;
+  const double *done = c->iter_ctl.first ? nullptr : scal + SC_DONE;
   // XArgs.scal serves only the mean of rhs, read at SC_SUM_RHS: point it so
   // that slot is sum_slot
   XArgs xa{g, P, rho_new, rhs, scal + (sum_slot - SC_SUM_RHS), c->spec[0], c->tw[0], (double)g.n, done, res};
@@ -1698,7 +1703,7 @@ void launch_poisson_iteration_on(tpx_ctx *c, const double *rho_new, double *P, c
   // residual goes through the five-pass kernels
   if (!res && three_pass_shape(c, r1, r2, y1, y2, z1, z2)) {
     const unsigned nb13 = three_pass_launch(c, xa, xi, done, r1, r2, y1, y2);
-    tpx_launch<k_finish_iter>(1, 1024, 0, c->stream, c->partials, nb13, scal, c->Iteration, c->p.epsilon);
+    tpx_launch<k_finish_iter>(1, 1024, 0, c->stream, c->partials, nb13, scal, c->Iteration, c->p.epsilon, c->iter_ctl);
     TPX_LAUNCH_CHECK();
     timing_end(c, TPX_K_FFT_INV);
     return;
@@ -1773,7 +1778,7 @@ void launch_poisson_iteration_on(tpx_ctx *c, const double *rho_new, double *P, c
     tpx_launch<k_xinv>(nbx, kThreads, shx, c->stream, xi, cx);
   }
   TPX_LAUNCH_CHECK();
-  tpx_launch<k_finish_iter>(1, 1024, 0, c->stream, c->partials, nbx, scal, c->Iteration, c->p.epsilon);
+  tpx_launch<k_finish_iter>(1, 1024, 0, c->stream, c->partials, nbx, scal, c->Iteration, c->p.epsilon, c->iter_ctl);
   TPX_LAUNCH_CHECK();
   timing_end(c, TPX_K_FFT_INV);
 }
@@ -1788,13 +1793,13 @@ void launch_coef_iteration(tpx_ctx *c, const double *const cf[3], double *P, con
   const Geo &g = c->g;
   int r1, r2, y1, y2, z1, z2;
   if (three_pass_shape(c, r1, r2, y1, y2, z1, z2)) {
-    const double *done = c->scal + SC_DONE;
+    const double *done = c->iter_ctl.first ? nullptr : c->scal + SC_DONE;
     timing_begin(c, TPX_K_FFT);
     XArgs xa{g, P, nullptr, rhs, c->scal, c->spec[0], c->tw[0], (double)g.n, done, nullptr};
     for (int d = 0; d < 3; ++d) xa.cf[d] = cf[d];
     const XInvArgs xi{g, P, c->spec[0], c->tw[0], c->partials, (double)g.n, done};
     const unsigned nb13 = three_pass_launch(c, xa, xi, done, r1, r2, y1, y2);
-    tpx_launch<k_finish_iter>(1, 1024, 0, c->stream, c->partials, nb13, c->scal, c->Iteration, c->p.epsilon);
+    tpx_launch<k_finish_iter>(1, 1024, 0, c->stream, c->partials, nb13, c->scal, c->Iteration, c->p.epsilon, c->iter_ctl);
     TPX_LAUNCH_CHECK();
     timing_end(c, TPX_K_FFT_INV);
     return;

@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <initializer_list>
 #include <memory>
 #include <mutex>
@@ -398,33 +399,70 @@ void do_update_ru_wop(tpx_ctx *c, int rk, bool with_rho) {
                 with_rho ? c->rho[c->rho_np1] : nullptr, with_rho ? c->rho[c->rho_new] : nullptr);
 }
 
-// Solve_Poisson's loop (poisson.cpp:391-462).  The loop test runs on the
-// device after every iteration, and iterations queued after it fails skip
-// themselves, so the host queues iterations in batches and waits once per
-// batch instead of once per iteration: first as many as the last solve of
-// this substep took, then two at a time.
-// The host side of every Poisson solve: the device counts the iterations and
-// evaluates the stopping rule (poisson.cpp:397) itself, so iterations are
-// queued in batches (the first as long as `guess`, then two at a time) and
-// the host waits once per batch.  Returns the iterations that ran.
+// Waits until the running solve has stopped or finished `want` iterations;
+// returns the iterations finished, and whether it has stopped.  The loop state
+// is read from pinned memory that the device writes after every iteration: the
+// next launch follows a couple of microseconds after the solve ends, where a
+// copy of the state and a stream wait, once per two iterations, left the GPU
+// idle (a 12-iteration solve at 32^3 401 -> 250-285 us, 13 at 128^3 906 ->
+// 820-846; 40 steps at 32^3 with two iterations a solve 21.4 -> 16.4 ms).  A
+// solve that takes long enough for that not to matter is waited for on the
+// stream.
+int wait_iterations(tpx_ctx *c, int want, bool &stopped) {
+  auto state = [&](int &its) {
+    const uint64_t v = __atomic_load_n(c->h_iter, __ATOMIC_ACQUIRE);
+    if ((uint32_t)(v >> 32) != c->solve_epoch) return false;
+    its = (int)((v & 0xffffffffu) >> 1);
+    stopped = v & 1;
+    return stopped || its >= want;
+  };
+  int its = 0;
+  const auto t0 = std::chrono::steady_clock::now();
+  do {
+    for (int q = 0; q < 64; ++q) {
+      if (state(its)) return its;
+      __builtin_ia32_pause();
+    }
+  } while (std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(300));
+  sync(c);
+  if (!state(its)) throw std::runtime_error("a Poisson iteration left no loop state");
+  return its;
+}
+
+// The host side of every Poisson solve (Solve_Poisson's loop,
+// poisson.cpp:391-462).  The device counts the iterations and evaluates the
+// stopping rule (poisson.cpp:397) itself, and an iteration queued after the
+// solve has stopped skips itself, so the host need not wait for each: it
+// queues `guess` iterations, and while the solve has not stopped then, two
+// more and one for each that ends.  Returns the iterations that ran.
 int solve_loop(tpx_ctx *c, int guess, const std::function<void(int)> &iterate) {
-  launch_solve_begin(c);
-  int queued = 0, batch = std::max(1, guess);
-  double st[2] = {0.0, 1.0};  // SC_ITERS, SC_DONE
-  while (queued < c->Iteration) {
-    const int nb = std::min(batch, c->Iteration - queued);
-    for (int b = 0; b < nb; ++b) iterate(queued + b);
-    queued += nb;
-    hip_check(hipMemcpyAsync(c->h_scal + SC_ITERS, c->scal + SC_ITERS, 2 * sizeof(double), hipMemcpyDeviceToHost,
-                             c->stream),
-              "hipMemcpyAsync");
-    sync(c);
-    st[0] = c->h_scal[SC_ITERS];
-    st[1] = c->h_scal[SC_DONE];
-    if (st[1] != 0.0) break;
-    batch = 2;
+  if (!(0 < c->Iteration && 100.0 > c->p.epsilon)) {  // err = 100 before the first (poisson.cpp:391-396)
+    launch_solve_begin(c);
+    return 0;
   }
-  return (int)st[0];
+  struct Running {  // the iterations of this solve report to the host
+    tpx_ctx *c;
+    explicit Running(tpx_ctx *ctx) : c(ctx) {
+      c->iter_ctl = {1, ++c->solve_epoch, c->h_iter};
+    }
+    ~Running() { c->iter_ctl = {}; }
+  } running(c);
+  int queued = 0;
+  auto queue = [&](int n) {
+    for (; n > 0 && queued < c->Iteration; --n) {
+      iterate(queued++);
+      c->iter_ctl.first = 0;
+    }
+  };
+  queue(std::max(1, guess));
+  bool stopped = false;
+  int its = wait_iterations(c, queued, stopped);
+  if (!stopped) queue(1);
+  while (!stopped) {  // the iteration count stops it at the latest
+    queue(1);
+    its = wait_iterations(c, std::max(its + 1, queued - 1), stopped);
+  }
+  return its;
 }
 
 void do_solve_poisson(tpx_ctx *c, int rk, int *iters, const std::function<void(int)> &before_iteration = {}) {
@@ -441,7 +479,8 @@ void do_solve_poisson(tpx_ctx *c, int rk, int *iters, const std::function<void(i
 // poisson::FFT with the caller's face coefficient (poisson.cpp:391-411).  P,
 // RHS, C and res (work) are dense device arrays.
 void do_solve_coef(tpx_ctx *c, const double *const cf[3], double *P, const double *rhs, double *res, int *iters) {
-  const int i = solve_loop(c, 2, [&](int) { launch_coef_iteration(c, cf, P, rhs, res); });
+  const int i = solve_loop(c, c->coef_guess, [&](int) { launch_coef_iteration(c, cf, P, rhs, res); });
+  c->coef_guess = i;
   c->num_iteration = i;  // the reference's poisson object keeps the last solve's count
   if (iters) *iters = i;
 }
@@ -465,11 +504,12 @@ void do_compute_rhs_pois_q(tpx_ctx *c, int rk) {
 // grid::Solve_Poisson_Q (grid.cpp:703-707): the FFT iteration with the
 // constant density Rho_forV; the solver's iteration count is shared with the
 // gas's solve, as the reference's single poisson object is
-void do_solve_poisson_q(tpx_ctx *c, int *iters) {
+void do_solve_poisson_q(tpx_ctx *c, int rk, int *iters) {
   ensure_passive_vector(c);
-  const int i = solve_loop(c, 2, [&](int) {
+  const int i = solve_loop(c, c->vec_guess[rk & 3], [&](int) {
     launch_poisson_iteration_on(c, c->rho_forv_field, c->Qv, c->rhs_q, c->scal, nullptr, SC_SUM_RHS_Q);
   });
+  c->vec_guess[rk & 3] = i;
   c->num_iteration = i;
   if (iters) *iters = i;
 }
@@ -483,7 +523,7 @@ void do_update_rv_wq(tpx_ctx *c, int rk) {
 void do_passive_vector(tpx_ctx *c, int rk) {
   do_update_rv_woq(c, rk);
   do_compute_rhs_pois_q(c, rk);
-  do_solve_poisson_q(c, nullptr);
+  do_solve_poisson_q(c, rk, nullptr);
   do_update_rv_wq(c, rk);
 }
 
@@ -659,6 +699,7 @@ void release(tpx_ctx *c) {
   for (auto &p : c->ps) f(p);
   adjoint_free(c->adj);
   if (c->h_scal) (void)hipHostFree(c->h_scal);
+  if (c->h_iter) (void)hipHostFree(c->h_iter);
   for (int t = 0; t < kStageMaxThreads; ++t) {
     if (c->stage.pin[t]) (void)hipHostFree(c->stage.pin[t]);
     for (hipEvent_t e : c->stage.ev[t])
@@ -795,6 +836,9 @@ int tpx_create(const tpx_params *p, int64_t np_capacity, tpx_ctx **out) {
     if (hipHostMalloc((void **)&c->h_scal, sizeof(double) * SC_COUNT, hipHostMallocDefault) != hipSuccess)
       throw std::bad_alloc();
     memset(c->h_scal, 0, sizeof(double) * SC_COUNT);
+    if (hipHostMalloc((void **)&c->h_iter, sizeof(uint64_t), hipHostMallocCoherent) != hipSuccess)
+      throw std::bad_alloc();
+    *c->h_iter = 0;
     hip_check(hipMemset(c->scal, 0, sizeof(double) * SC_COUNT), "hipMemset");
     for (auto &f : c->S) hip_check(hipMemset(f, 0, sizeof(double) * n), "hipMemset");
     hip_check(hipMemset(c->Q, 0, sizeof(double) * n), "hipMemset");
@@ -1101,7 +1145,7 @@ int tpx_solve_poisson_q(tpx_ctx *ctx, int rk, int *iterations) {
   return guarded(ctx, [&]() {
     TPX_RK_CHECK(rk);
     if (!ctx->p.solve_for_vector) throw std::logic_error("Solve_Poisson_Q with solve_for_vector = 0");
-    do_solve_poisson_q(ctx, iterations);
+    do_solve_poisson_q(ctx, rk, iterations);
     return TPX_OK;
   });
 }
@@ -1692,9 +1736,9 @@ void gas_substeps(tpx_ctx *c, int s, GasSubstep sub[4], bool segment) {
     // count the device's loop test reaches is kept for a check after the
     // sweep (the replay is the recorded run bit for bit, so no iteration is
     // skipped on the device before the recorded count)
-    launch_solve_begin(c);
     g.P.clear();
     g.iters = t.iters[q];
+    if (g.iters == 0) launch_solve_begin(c);
     if (segment) t.p_first[q] = used;
     for (int it = 0; it < g.iters; ++it) {
       double *buf = pcap_slot(t, used++, n);
@@ -1703,7 +1747,9 @@ void gas_substeps(tpx_ctx *c, int s, GasSubstep sub[4], bool segment) {
       g.P.push_back(buf);
       double *out = c->P;
       if (it + 1 < g.iters && !(out = pcap_slot(t, used, n))) throw std::bad_alloc();
+      c->iter_ctl.first = it == 0;
       launch_poisson_iteration_on(c, c->rho[c->rho_new], buf, c->rhs, c->scal, nullptr, SC_SUM_RHS, out);
+      c->iter_ctl.first = 0;
     }
     launch_copy(c, t.iters_seen + (long)s * 4 + rk, c->scal + SC_ITERS, 1);
     do_update_ru_wp(c, rk, rk == 3);

@@ -27,6 +27,20 @@
 
 namespace tpx {
 
+// A pointer read from an argument table is a generic (flat) address to the
+// compiler, where a kernel's own pointer argument is known to be global: its
+// accesses become flat loads and stores, which also count against the LDS
+// wait counter, so every LDS wait of the body waits on them too.  Every table
+// pointer is device (or pinned host) memory: gptr hands it on as a global
+// pointer (the empty asm keeps the compiler from folding the two casts away),
+// and the accesses compile as for a kernel argument.  An argument struct with
+// a to_global() member has its pointers passed through gptr the same way.
+template <class V>
+__device__ __forceinline__ V *gptr(V *p) {
+  __attribute__((address_space(1))) V *g = (__attribute__((address_space(1))) V *)p;
+  asm("" : "+s"(g));
+  return (V *)g;
+}
 // device scalar slots (ctx->scal)
 enum Scal {
   SC_P0 = 0, SC_P0_INT, SC_P0_NEW, SC_P0_NP1, SC_DP0_DT, SC_MET,  // Update_P0 state
@@ -230,6 +244,17 @@ struct HostStage {
   int threads = 0;
 };
 
+// How a Poisson iteration takes part in its solve's loop: `first` iterations
+// run without reading the loop test (and restart the count), and `host`, if
+// set, is pinned memory that receives epoch << 32 | iterations << 1 | stopped
+// after each one.
+struct IterCtl {
+  int first = 0;
+  uint32_t epoch = 0;
+  uint64_t *host = nullptr;
+  __device__ void to_global() { host = gptr(host); }
+};
+
 struct Timing {
   bool on = false;
   struct Rec { int cls; hipEvent_t a, b; };
@@ -253,6 +278,11 @@ struct tpx_ctx {
   int num_iteration = 0;
   int64_t total_iterations = 0;    // summed over all Poisson solves
   int iter_guess[4] = {4, 4, 4, 4}; // iterations queued up front, per substep (last solve's count)
+  int coef_guess = 4;              // the same for a solve with the caller's coefficient
+  int vec_guess[4] = {2, 2, 2, 2}; // and for the passive vector's
+  tpx::IterCtl iter_ctl;           // of the iteration being launched
+  uint64_t *h_iter = nullptr;      // pinned, coherent: the loop state of the running solve
+  uint32_t solve_epoch = 0;
   hipStream_t stream = nullptr;
   int device = 0;
   size_t max_lds = 65536;          // dynamic LDS bytes one workgroup may use on this device
@@ -490,20 +520,6 @@ __device__ __forceinline__ unsigned block_dim_x() {
   return *(const uint16_t *)((const char *)__builtin_amdgcn_implicitarg_ptr() + 12);
 }
 
-// A pointer read from an argument table is a generic (flat) address to the
-// compiler, where a kernel's own pointer argument is known to be global: its
-// accesses become flat loads and stores, which also count against the LDS
-// wait counter, so every LDS wait of the body waits on them too.  Every table
-// pointer is device (or pinned host) memory: gptr hands it on as a global
-// pointer (the empty asm keeps the compiler from folding the two casts away),
-// and the accesses compile as for a kernel argument.  An argument struct with
-// a to_global() member has its pointers passed through gptr the same way.
-template <class V>
-__device__ __forceinline__ V *gptr(V *p) {
-  __attribute__((address_space(1))) V *g = (__attribute__((address_space(1))) V *)p;
-  asm("" : "+s"(g));
-  return (V *)g;
-}
 template <class V, class = void>
 struct has_to_global : std::false_type {};
 template <class V>
