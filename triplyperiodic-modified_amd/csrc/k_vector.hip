@@ -2,11 +2,13 @@
 // a momentum-like field RV at the faces, transported by the gas velocity
 // U = RU_int/Rho_face, diffused with eta, forced by V_Source (or by the gas's
 // x velocity on its y component), and projected with its own pressure Q
-// (a Poisson solve with the constant density Rho_forV).  One thread per
-// cell; every product and sum in the order of the reference's whole-array
-// passes (built with -ffp-contract=off), so the stencil parts round as the
-// reference's do.
+// (a Poisson solve with the constant density Rho_forV).  Every product and sum
+// in the order of the reference's whole-array passes (built with
+// -ffp-contract=off), so the stencil parts round as the reference's do.
 #include <math.h>
+
+#include <algorithm>
+#include <stdexcept>
 
 #include "tpx_internal.h"
 
@@ -57,71 +59,158 @@ struct RvArgs {
   int s2_type, rk3;
 };
 
-// grid::Update_RV_WOQ (grid.cpp:646-692) at the three faces of one cell
+// grid::Update_RV_WOQ (grid.cpp:646-692) as a z-marching tile.  Evaluated a
+// thread a cell from global memory, every face reads up to 60 neighbours and
+// forms V = RV_int/Rho_forV and U = RU_int/Rho_face anew at each (some 70
+// divisions a cell): bound by address processing and divisions, 241 us at
+// 128^3 against a floor of 70 us for its 19 field values a cell.  A block owns
+// a TX x TY column and walks KC planes: RV_int, V and U of the planes k and
+// k + 1 (one halo cell on each side; the divisions are done once, as a point is
+// loaded) lie in LDS, the own column's values of plane k - 1 in registers, and
+// the plane after next is loaded while this one is computed: 113 us.  49 KB of
+// LDS a block of 256, three blocks a CU.  Same operands and order: the same
+// bits.
+struct RvTile { int TX, TY, KC; };
+
 struct k_rv_woq {
   static constexpr int kBounds = 256;
-  static __device__ __forceinline__ void run(const Geo &g, const RvArgs &a) {
-    int i, j, k;
-    long c;
-    if (!cell(g, i, j, k, c)) return;
+  static __device__ __forceinline__ void run(const Geo &g, const RvArgs &a, const RvTile &tl) {
+    extern __shared__ double sm[];
+    const int TX = tl.TX, TY = tl.TY, KC = tl.KC;
+    const int TW = TX + 2, TN = TW * (TY + 2);  // x from i0 - 1 to i0 + TX
     const IxV ix = ixv(g);
-    const double id[3] = {g.idx, g.idy, g.idz}, id2[3] = {g.idx2, g.idy2, g.idz2};
-    const int e[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
-    auto at = [&](int di, int dj, int dk) { return ix(i + di, j + dj, k + dk); };
-    // V = RV_int / Rho_forV (tensor0.cpp:143-147)
-    auto V = [&](int b, long q) { return a.rv_int[b][q] / a.rho_forv; };
-    // div_F2C(V) at the cell offset by (di, dj, dk) (tensor0.cpp:249-256)
-    auto divV = [&](int di, int dj, int dk) {
-      const long q = at(di, dj, dk);
-      return (V(0, at(di + 1, dj, dk)) - V(0, q)) * g.idx + (V(1, at(di, dj + 1, dk)) - V(1, q)) * g.idy +
-             (V(2, at(di, dj, dk + 1)) - V(2, q)) * g.idz;
-    };
-    // U.d = RU_int.d / Rho_face.d, Rho_face = I_C2F(Rho_int) (grid.cpp:868)
-    auto U = [&](int d, long q, int di, int dj, int dk) {
-      const long qm = at(di - e[d][0], dj - e[d][1], dk - e[d][2]);
-      return a.ru_int[d][q] / ((a.rho_int[q] + a.rho_int[qm]) * 0.5);
-    };
-    const double div0 = divV(0, 0, 0);
-    for (int ax = 0; ax < 3; ++ax) {
-      const int* ea = e[ax];
-      const double g1 = (div0 - divV(-ea[0], -ea[1], -ea[2])) * id[ax];  // grad_C2F (tensor1.cpp:259-270)
-      double lap = 0.0;                                                  // del2 (tensor0.cpp:258-266)
+    const unsigned b = xcd_block(blockIdx.x, gridDim.x);
+    const int ntx = g.nx / TX, nty = g.ny / TY;
+    const int i0 = (int)(b % ntx) * TX, j0 = (int)((b / ntx) % nty) * TY, k0 = (int)(b / (ntx * nty)) * KC;
+    const int tid = (int)threadIdx.x, bd = (int)block_dim_x(), tx = tid % TX, ty = tid / TX;
+    const int i = i0 + tx, j = j0 + ty;
+    const double *__restrict__ rho = a.rho_int;
+    // one point of a plane as loaded: RV_int, RU_int, Rho at the point and below it
+    struct Raw { double rv[3], ru[3], r[4]; };
+    auto load = [&](int kz, int e, Raw &w) {
+      const int x = i0 + e % TW - 1, y = j0 + e / TW - 1;
+      const long q = ix(x, y, kz);
+#pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const double l = (V(ax, at(e[d][0], e[d][1], e[d][2])) - 2 * V(ax, c) + V(ax, at(-e[d][0], -e[d][1], -e[d][2]))) *
-                         id2[d];
-        lap = d == 0 ? l : lap + l;
+        w.rv[d] = a.rv_int[d][q];
+        w.ru[d] = a.ru_int[d][q];
       }
-      double rhs = a.eta / 3. * g1 + a.eta * lap;
-      // convection: div_F2C of I_d(RV_int.ax) * I_ax(U.d) (grid.cpp:655-673)
-      double conv = 0.0;
+      w.r[0] = rho[q];
+      w.r[1] = rho[ix(x - 1, y, kz)];
+      w.r[2] = rho[ix(x, y - 1, kz)];
+      w.r[3] = rho[ix(x, y, kz - 1)];
+    };
+    // V = RV_int/Rho_forV (tensor0.cpp:143-147), U.d = RU_int.d/Rho_face.d with
+    // Rho_face = I_C2F(Rho_int) (grid.cpp:868)
+    auto store = [&](const Raw &w, int slot, int e) {
+      double *t = sm + slot * 9 * TN + e;
+#pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const int *ed = e[d];
-        // the two faces of direction d around the cell: q0 = the cell, q1 = the cell + e_d
-        double T[2];
-        for (int s = 0; s < 2; ++s) {
-          const int oi = s * ed[0], oj = s * ed[1], ok = s * ed[2];
-          const long q = at(oi, oj, ok);
-          const double irv = (a.rv_int[ax][q] + a.rv_int[ax][at(oi - ed[0], oj - ed[1], ok - ed[2])]) * 0.5;
-          const double iu = (U(d, q, oi, oj, ok) +
-                             U(d, at(oi - ea[0], oj - ea[1], ok - ea[2]), oi - ea[0], oj - ea[1], ok - ea[2])) * 0.5;
-          T[s] = irv * iu;
-        }
-        const double t = (T[1] - T[0]) * id[d];
-        conv = d == 0 ? t : conv + t;
+        t[d * TN] = w.rv[d];
+        t[(3 + d) * TN] = w.rv[d] / a.rho_forv;
+        t[(6 + d) * TN] = w.ru[d] / ((w.r[0] + w.r[1 + d]) * 0.5);
       }
-      rhs -= conv;
+    };
+    // a plane is at most two points a thread: (TX + 2)(TY + 2) <= 2 TX TY
+    auto load_plane = [&](int kz, Raw (&w)[2]) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (tid + u * bd < TN) load(kz, tid + u * bd, w[u]);
+    };
+    auto store_plane = [&](const Raw (&w)[2], int slot) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (tid + u * bd < TN) store(w[u], slot, tid + u * bd);
+    };
+    // quantity q (0-2 RV_int, 3-5 V, 6-8 U) of slot s at cell (i + dx, j + dy)
+    auto T = [&](int s, int q, int dx, int dy) -> double {
+      return sm[(s * 9 + q) * TN + (ty + 1 + dy) * TW + tx + 1 + dx];
+    };
+    // div_F2C(V) at (i + dx, j + dy) of plane `s`, the plane above in slot `n` (tensor0.cpp:249-256)
+    auto divV = [&](int s, int n, int dx, int dy) {
+      return (T(s, 3, dx + 1, dy) - T(s, 3, dx, dy)) * g.idx + (T(s, 4, dx, dy + 1) - T(s, 4, dx, dy)) * g.idy +
+             (T(n, 5, dx, dy) - T(s, 5, dx, dy)) * g.idz;
+    };
+    Raw w[2];
+    load_plane(k0 - 1, w);
+    store_plane(w, 1);
+    load_plane(k0, w);
+    store_plane(w, 0);
+    load_plane(k0 + 1, w);
+    __syncthreads();
+    // own-column values of the plane below
+    double RVp[3], Vp[3], Uxp, Uxp1, Uyp, Uyp1, Uzp, dvp;
+    auto carry = [&](int s, int n) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        RVp[d] = T(s, d, 0, 0);
+        Vp[d] = T(s, 3 + d, 0, 0);
+      }
+      Uxp = T(s, 6, 0, 0);
+      Uxp1 = T(s, 6, 1, 0);
+      Uyp = T(s, 7, 0, 0);
+      Uyp1 = T(s, 7, 0, 1);
+      Uzp = T(s, 8, 0, 0);
+      dvp = divV(s, n, 0, 0);
+    };
+    carry(1, 0);
+    __syncthreads();
+    store_plane(w, 1);
+    __syncthreads();
+    const double id[3] = {g.idx, g.idy, g.idz};
+    int cur = 0;
+    for (int kk = k0; kk < k0 + KC; ++kk) {
+      const int nxt = cur ^ 1;
+      const bool more = kk + 1 < k0 + KC;
+      if (more) load_plane(kk + 2, w);
+      const long c = (long)kk * g.nxy + (long)j * g.nx + i;
+      const double div0 = divV(cur, nxt, 0, 0);
+      double s2[3] = {0.0, 0.0, 0.0};
       if (a.s2_type == 0) {
         // V_Source (grid.cpp:616-641, vector_source.h): cos(X) on the y faces,
         // zero on the others, each minus its mean over the cells
         const double X = i * g.dx + g.dx / 2., A = 1., K = 1.;
-        const double s2 = ax == 1 ? A * cos(K * X) - a.scal[SC_RV_S2] / a.ncell : 0.0;
-        rhs += s2;
-      } else if (ax == 1) {
-        rhs += -1 * a.filt[c];
+        s2[1] = A * cos(K * X) - a.scal[SC_RV_S2] / a.ncell;
+      } else {
+        s2[1] = -1 * a.filt[c];
       }
-      const double np1 = a.rv_np1[ax][c] + a.c_post * rhs;
-      a.rv_np1[ax][c] = np1;
-      a.rv_new[ax][c] = a.rk3 ? np1 : 1 * a.rv_base[ax][c] + a.c_pre * rhs;
+#pragma unroll
+      for (int ax = 0; ax < 3; ++ax) {
+        const int ei = ax == 0, ej = ax == 1;
+        const bool ez = ax == 2;
+        const double dvm = ez ? dvp : divV(cur, nxt, -ei, -ej);
+        const double g1 = (div0 - dvm) * id[ax];  // grad_C2F (tensor1.cpp:259-270)
+        const double vc = T(cur, 3 + ax, 0, 0);
+        // del2 (tensor0.cpp:258-266)
+        double lap = (T(cur, 3 + ax, 1, 0) - 2 * vc + T(cur, 3 + ax, -1, 0)) * g.idx2;
+        lap = lap + (T(cur, 3 + ax, 0, 1) - 2 * vc + T(cur, 3 + ax, 0, -1)) * g.idy2;
+        lap = lap + (T(nxt, 3 + ax, 0, 0) - 2 * vc + Vp[ax]) * g.idz2;
+        double rhs = a.eta / 3. * g1 + a.eta * lap;
+        // convection: div_F2C of I_d(RV_int.ax) * I_ax(U.d) (grid.cpp:655-673)
+        const double rc = T(cur, ax, 0, 0);
+        const double ux0 = ((rc + T(cur, ax, -1, 0)) * 0.5) * ((T(cur, 6, 0, 0) + (ez ? Uxp : T(cur, 6, -ei, -ej))) * 0.5);
+        const double ux1 =
+            ((T(cur, ax, 1, 0) + rc) * 0.5) * ((T(cur, 6, 1, 0) + (ez ? Uxp1 : T(cur, 6, 1 - ei, -ej))) * 0.5);
+        const double uy0 = ((rc + T(cur, ax, 0, -1)) * 0.5) * ((T(cur, 7, 0, 0) + (ez ? Uyp : T(cur, 7, -ei, -ej))) * 0.5);
+        const double uy1 =
+            ((T(cur, ax, 0, 1) + rc) * 0.5) * ((T(cur, 7, 0, 1) + (ez ? Uyp1 : T(cur, 7, -ei, 1 - ej))) * 0.5);
+        const double uz0 = ((rc + RVp[ax]) * 0.5) * ((T(cur, 8, 0, 0) + (ez ? Uzp : T(cur, 8, -ei, -ej))) * 0.5);
+        const double uz1 = ((T(nxt, ax, 0, 0) + rc) * 0.5) *
+                           ((T(nxt, 8, 0, 0) + (ez ? T(cur, 8, 0, 0) : T(nxt, 8, -ei, -ej))) * 0.5);
+        double conv = (ux1 - ux0) * g.idx;
+        conv = conv + (uy1 - uy0) * g.idy;
+        conv = conv + (uz1 - uz0) * g.idz;
+        rhs -= conv;
+        if (a.s2_type == 0 || ax == 1) rhs += s2[ax];
+        const double np1 = a.rv_np1[ax][c] + a.c_post * rhs;
+        a.rv_np1[ax][c] = np1;
+        a.rv_new[ax][c] = a.rk3 ? np1 : 1 * a.rv_base[ax][c] + a.c_pre * rhs;
+      }
+      carry(cur, nxt);
+      __syncthreads();
+      if (more) store_plane(w, cur);
+      cur = nxt;
+      __syncthreads();
     }
   }
 };
@@ -248,7 +337,19 @@ void launch_rv_woq(tpx_ctx *c, const Coef &k, const double *const ru_int[3], con
     TPX_LAUNCH_CHECK();
     a.filt = c->rv_filt;
   }
-  tpx_launch<k_rv_woq>(vgrid(c), 256, 0, c->stream, c->g, a);
+  const Geo &g = c->g;
+  RvTile tl;
+  tl.TX = std::min(g.nx, 32);
+  tl.TY = std::min(256 / tl.TX, g.ny);
+  // a march of up to 16 planes, shorter while the launch has fewer than 1024
+  // blocks (the two halo planes re-read by each block cost less than idle CUs)
+  tl.KC = std::min(g.nz, 16);
+  const int cols = (g.nx / tl.TX) * (g.ny / tl.TY);
+  while (tl.KC > 2 && cols * (g.nz / tl.KC) < 1024) tl.KC /= 2;
+  const int tile = (tl.TX + 2) * (tl.TY + 2);
+  if (tile > 2 * tl.TX * tl.TY) throw std::logic_error("passive vector tile exceeds two points per thread");
+  tpx_launch<k_rv_woq>((unsigned)(cols * (g.nz / tl.KC)), tl.TX * tl.TY, sizeof(double) * 18 * (size_t)tile, c->stream,
+                       g, a, tl);
   TPX_LAUNCH_CHECK();
   timing_end(c, TPX_K_OTHER);
 }
