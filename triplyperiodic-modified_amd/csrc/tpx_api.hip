@@ -211,83 +211,93 @@ bool is_vector(int field) { return field >= TPX_RU && field <= TPX_RV_NP1; }
 
 void sync(tpx_ctx *c) { hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize"); }
 
-// ---- device to host ------------------------------------------------------
+// ---- host to device and back ---------------------------------------------
 struct HostPart {
   void *dst;
   const void *src;
   size_t bytes;
 };
 
-// The staging of a context, made on its first download: a pinned pair of
-// chunks and their events per copying thread.  Without it (no pinned memory
-// left) the runtime's own pageable copy serves.
-bool stage_ready(tpx_ctx *c, int threads) {
+// The staging of a context: a pinned pair of chunks and their events per
+// copying thread, the first thread's pair allocated with the context, the
+// others on the first transfer that uses them.  Without more pinned memory
+// fewer threads copy.
+void stage_ready(tpx_ctx *c, int threads) {
   HostStage &st = c->stage;
   while (st.threads < threads) {
     const int t = st.threads;
-    if (hipHostMalloc((void **)&st.pin[t], 2 * kStageChunk, hipHostMallocDefault) != hipSuccess) {
+    if (t > 0 && hipHostMalloc((void **)&st.pin[t], 2 * st.chunk, hipHostMallocDefault) != hipSuccess) {
       (void)hipGetLastError();
       st.pin[t] = nullptr;
-      return t > 0;
+      return;
     }
     for (int e = 0; e < 2; ++e)
       hip_check(hipEventCreateWithFlags(&st.ev[t][e], hipEventDisableTiming), "hipEventCreate");
     st.threads = t + 1;
   }
-  return true;
 }
 
-// Copies device arrays into the caller's host arrays, in order after the
-// context's queued work, and returns when they are there.  Bound by the
-// caller's side, not by the link: into fresh pages (134 MB) the runtime's
+// Copies between the caller's host arrays and device arrays, in order after
+// the context's queued work, and returns when the data are there.  Bound by
+// the caller's side, not by the link: into fresh pages (134 MB) the runtime's
 // pageable copy takes 13-45 ms, the link alone 2.4 ms (56 GB/s).  The arrays
 // are taken in 1 MiB chunks through pinned pairs, one chunk crossing the link
-// while the last is copied out, on four threads (which also share the page
+// while the host copies another, on four threads (which also share the page
 // faults) from 8 MiB up: 4.5-5.6 ms; more threads or larger chunks were
 // slower (8 threads 6.6, 4 MiB chunks 6.9).
-void download(tpx_ctx *c, const HostPart *part, int nparts) {
+void transfer(tpx_ctx *c, const HostPart *part, int nparts, bool up) {
   struct Piece {
     char *dst;
     const char *src;
     size_t bytes;
   };
+  const hipMemcpyKind kind = up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
+  const char *what = up ? "upload" : "download";
+  const size_t chunk = c->stage.chunk;
   std::vector<Piece> pieces;
   size_t total = 0;
   for (int q = 0; q < nparts; ++q) {
     total += part[q].bytes;
-    for (size_t o = 0; o < part[q].bytes; o += kStageChunk)
-      pieces.push_back({(char *)part[q].dst + o, (const char *)part[q].src + o, std::min(kStageChunk, part[q].bytes - o)});
+    for (size_t o = 0; o < part[q].bytes; o += chunk)
+      pieces.push_back({(char *)part[q].dst + o, (const char *)part[q].src + o, std::min(chunk, part[q].bytes - o)});
   }
   if (pieces.empty()) return sync(c);
   int threads = total >= (8u << 20) ? kStageMaxThreads : 1;
-  if (!stage_ready(c, threads)) {
-    for (const Piece &p : pieces)
-      hip_check(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, c->stream), "download");
-    return sync(c);
-  }
+  stage_ready(c, threads);
   threads = std::min(threads, c->stage.threads);
   std::atomic<size_t> next{0};
   std::atomic<int> failed{(int)hipSuccess};
   auto work = [&](int t) {
     HostStage &st = c->stage;
-    char *slot[2] = {st.pin[t], st.pin[t] + kStageChunk};
+    char *slot[2] = {st.pin[t], st.pin[t] + chunk};
     hipError_t e = t > 0 ? hipSetDevice(c->device) : hipSuccess;  // a helper starts on device 0
-    size_t held[2] = {pieces.size(), pieces.size()};  // the piece in flight to each slot
+    const size_t none = pieces.size();
+    size_t held[2] = {none, none};  // the piece in flight through each slot
+    // waits for the slot's piece; a downloaded one goes to its place
+    auto drain = [&](int k) {
+      if (e != hipSuccess || held[k] == none) return;
+      e = hipEventSynchronize(st.ev[t][k]);
+      if (e == hipSuccess && !up) memcpy(pieces[held[k]].dst, slot[k], pieces[held[k]].bytes);
+      held[k] = none;
+    };
     for (int k = 0; e == hipSuccess; k ^= 1) {
       const size_t i = next++;
-      if (i < pieces.size()) {
-        e = hipMemcpyAsync(slot[k], pieces[i].src, pieces[i].bytes, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipEventRecord(st.ev[t][k], c->stream);
-        if (e == hipSuccess) held[k] = i;
+      if (i >= none) break;
+      const Piece &p = pieces[i];
+      if (up) {
+        drain(k);
+        if (e != hipSuccess) break;
+        memcpy(slot[k], p.src, p.bytes);
+        e = hipMemcpyAsync(p.dst, slot[k], p.bytes, kind, c->stream);
+      } else {
+        e = hipMemcpyAsync(slot[k], p.src, p.bytes, kind, c->stream);
       }
-      const size_t j = held[k ^ 1];
-      if (e == hipSuccess && j < pieces.size()) {
-        e = hipEventSynchronize(st.ev[t][k ^ 1]);
-        if (e == hipSuccess) memcpy(pieces[j].dst, slot[k ^ 1], pieces[j].bytes);
-        held[k ^ 1] = pieces.size();
-      }
-      if (i >= pieces.size() && held[k] >= pieces.size()) break;
+      if (e == hipSuccess) e = hipEventRecord(st.ev[t][k], c->stream);
+      if (e == hipSuccess) held[k] = i;
+      if (!up) drain(k ^ 1);
     }
+    drain(0);
+    drain(1);
     if (e != hipSuccess) failed = (int)e;
   };
   std::vector<std::thread> helpers;
@@ -297,8 +307,11 @@ void download(tpx_ctx *c, const HostPart *part, int nparts) {
   }
   work(0);
   for (auto &h : helpers) h.join();
-  hip_check((hipError_t)failed.load(), "download");
+  hip_check((hipError_t)failed.load(), what);
 }
+
+void download(tpx_ctx *c, const HostPart *part, int nparts) { transfer(c, part, nparts, false); }
+void upload(tpx_ctx *c, const HostPart *part, int nparts) { transfer(c, part, nparts, true); }
 
 double read_scalar(tpx_ctx *c, int slot) {
   hip_check(hipMemcpyAsync(c->h_scal + slot, c->scal + slot, sizeof(double), hipMemcpyDeviceToHost, c->stream),
@@ -698,10 +711,9 @@ void release(tpx_ctx *c) {
   f(c->scal); f(c->partials); f(c->scan_tmp); f(c->st_part);
   for (auto &p : c->ps) f(p);
   adjoint_free(c->adj);
-  if (c->h_scal) (void)hipHostFree(c->h_scal);
-  if (c->h_iter) (void)hipHostFree(c->h_iter);
+  if (c->h_scal) (void)hipHostFree(c->h_scal);  // with h_iter and stage.pin[0]
   for (int t = 0; t < kStageMaxThreads; ++t) {
-    if (c->stage.pin[t]) (void)hipHostFree(c->stage.pin[t]);
+    if (t > 0 && c->stage.pin[t]) (void)hipHostFree(c->stage.pin[t]);
     for (hipEvent_t e : c->stage.ev[t])
       if (e) (void)hipEventDestroy(e);
   }
@@ -833,12 +845,20 @@ int tpx_create(const tpx_params *p, int64_t np_capacity, tpx_ctx **out) {
     c->n_partials = std::max((long)grid1d(g.n, 256), (long)g.ny * g.nz) + 1024;
     dalloc(&c->partials, 3 * (size_t)c->n_partials);
     ialloc(&c->scan_tmp, (size_t)(g.n / 2048 + 1024));
-    if (hipHostMalloc((void **)&c->h_scal, sizeof(double) * SC_COUNT, hipHostMallocDefault) != hipSuccess)
-      throw std::bad_alloc();
-    memset(c->h_scal, 0, sizeof(double) * SC_COUNT);
-    if (hipHostMalloc((void **)&c->h_iter, sizeof(uint64_t), hipHostMallocCoherent) != hipSuccess)
-      throw std::bad_alloc();
-    *c->h_iter = 0;
+    // one pinned block (each allocation costs some 0.3 ms here and as much
+    // again to free): the scalars' mirror, the solves' loop state on a line of
+    // its own, and the first copying thread's chunks
+    {
+      const size_t head = (sizeof(double) * SC_COUNT + 63) / 64 * 64, largest = sizeof(double) * std::max(n, (size_t)np_capacity);
+      c->stage.chunk = std::min(kStageChunk, (largest + 4095) / 4096 * 4096);
+      char *pin = nullptr;
+      if (hipHostMalloc((void **)&pin, head + 64 + 2 * c->stage.chunk, hipHostMallocCoherent) != hipSuccess)
+        throw std::bad_alloc();
+      memset(pin, 0, head + 64);
+      c->h_scal = (double *)pin;
+      c->h_iter = (uint64_t *)(pin + head);
+      c->stage.pin[0] = pin + head + 64;
+    }
     hip_check(hipMemset(c->scal, 0, sizeof(double) * SC_COUNT), "hipMemset");
     for (auto &f : c->S) hip_check(hipMemset(f, 0, sizeof(double) * n), "hipMemset");
     hip_check(hipMemset(c->Q, 0, sizeof(double) * n), "hipMemset");
@@ -906,8 +926,8 @@ int tpx_upload_field(tpx_ctx *ctx, int field, int comp, const double *host, int 
           memcpy(tmp.get() + ((size_t)k * g.ny + j) * g.nx, host + ((size_t)(k + bs) * GY + (j + bs)) * GX + bs,
                  sizeof(double) * g.nx);
     }
-    hip_check(hipMemcpyAsync(dst, bs > 0 ? tmp.get() : host, sizeof(double) * g.n, hipMemcpyHostToDevice, ctx->stream),
-              "upload");
+    const HostPart part{dst, bs > 0 ? tmp.get() : host, sizeof(double) * g.n};
+    upload(ctx, &part, 1);
     if (field == TPX_RHS_PART_TEMP) {
       launch_reduce(ctx, ctx->Q, 0, SC_SUM_Q);
       ctx->q_zero = false;
@@ -967,16 +987,17 @@ int tpx_upload_particles(tpx_ctx *ctx, int64_t n, const double *x, const double 
     pt.st_base = 0; pt.st_int = 1; pt.st_new = 2; pt.st_np1 = 3;
     pt.np1_is_base = true;
     pt.int_is_base = false;
-    for (int q = 0; q < 7; ++q)
-      if (n) hip_check(hipMemcpyAsync(pt.q[q][pt.st_base], src[q], sizeof(double) * n, hipMemcpyHostToDevice, ctx->stream), "upload");
-    if (n) hip_check(hipMemcpyAsync(pt.flag, flag, sizeof(int32_t) * n, hipMemcpyHostToDevice, ctx->stream), "upload");
     pt.has_tau = tau != nullptr;
     pt.has_eps = eps != nullptr;
-    if (tau && n) hip_check(hipMemcpyAsync(pt.tau, tau, sizeof(double) * n, hipMemcpyHostToDevice, ctx->stream), "upload");
-    if (eps && n) hip_check(hipMemcpyAsync(pt.eps, eps, sizeof(double) * n, hipMemcpyHostToDevice, ctx->stream), "upload");
+    HostPart part[10];
+    int m = 0;
+    for (int q = 0; q < 7; ++q) part[m++] = {pt.q[q][pt.st_base], src[q], sizeof(double) * (size_t)n};
+    part[m++] = {pt.flag, flag, sizeof(int32_t) * (size_t)n};
+    if (tau) part[m++] = {pt.tau, tau, sizeof(double) * (size_t)n};
+    if (eps) part[m++] = {pt.eps, eps, sizeof(double) * (size_t)n};
+    upload(ctx, part, m);
     pt.n = n;
     pt.new_counted = false;
-    sync(ctx);
     return TPX_OK;
   });
 }

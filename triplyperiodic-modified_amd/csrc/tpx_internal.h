@@ -234,14 +234,15 @@ struct TileTune {
   std::vector<Pending> pending;
 };
 
-// Pinned chunks that downloads pass through, and the events of the copies in
-// flight: two per copying thread, made on the first download that uses them.
-constexpr size_t kStageChunk = 1u << 20;
+// Pinned chunks that uploads and downloads pass through, and the events of the
+// copies in flight: two per copying thread.
+constexpr size_t kStageChunk = 1u << 20;  // largest chunk; a small context's holds its largest array
 constexpr int kStageMaxThreads = 4;
 struct HostStage {
   char *pin[kStageMaxThreads] = {};
   hipEvent_t ev[kStageMaxThreads][2] = {};
-  int threads = 0;
+  size_t chunk = kStageChunk;
+  int threads = 0;  // threads whose chunks and events exist
 };
 
 // How a Poisson iteration takes part in its solve's loop: `first` iterations
