@@ -752,7 +752,7 @@ void bin_positions(tpx_ctx *c, const double *Y, bool cic) {
   AdjointTape &t = c->adj;
   const long np = c->pt.n;
   launch_zero_counts(c, t.bstart);
-  tpx_launch<k_adj_bin_keys>(grid1(np), kBlock, 0, c->stream, c->g, Y, (int)cic, t.bkey, t.bstart, np);
+  tpx_launch<k_adj_bin_keys>(grid1(np), kBlock, 0, c->stream, c->g, Y, (int)cic, t.bkey, t.bstart + 1, np);
   TPX_LAUNCH_CHECK();
   launch_bin_by_key(c, t.bkey, t.bperm, t.binv, t.bstart);
 }

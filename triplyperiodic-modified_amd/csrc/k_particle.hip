@@ -70,7 +70,7 @@ struct AdvArgs {
   double *contrib;           // shares at sorted positions, 6 arrays (null: no two-way coupling)
   long cstride;
   const int32_t *inv_int;    // particle -> sorted position of x_int
-  int32_t *cnt;              // per-cell counts of x_new (null: no binning this substep)
+  int32_t *cnt;              // per-cell counts of x_new (start_new + 1) (null: no binning this substep)
   int32_t *key;
   long n;
   int int_is_base, np1_is_base;  // the int / np1 inputs are the base arrays
@@ -234,16 +234,8 @@ struct k_set_i {
 }
 };
 
-struct k_copy_i {
-  static constexpr int kBounds = 1024;
-  static __device__ __forceinline__ void run(int32_t *__restrict__ d, const int32_t *__restrict__ s, long n) {
-  long p = (long)blockIdx.x * block_dim_x() + threadIdx.x;
-  if (p < n) d[p] = s[p];
-}
-};
-
 // placement: each particle takes the next free slot of its cell's segment
-// (cursor starts as a copy of the CSR offsets).  The particles arrive nearly
+// (cursor[c]: the next free slot of cell c).  The particles arrive nearly
 // in cell order, so a wave's keys come in runs of equal cells on a few cache
 // lines, and returning atomics on one line are served one after another: each
 // run of equal keys in a wave reserves its slots with one atomic (taken by
@@ -329,50 +321,105 @@ struct k_iota {
 }
 };
 
-// ---- exclusive scan of int32 (three phases, block size 256 x 8) ----
-constexpr int kScanPer = 8;
-constexpr int kScanChunk = kBlock * kScanPer;
+// ---- exclusive scan of int32, in place, in two launches ----
+// A block takes `tiles` consecutive tiles of 4096 values: the first launch
+// leaves each block's total, the second adds up the totals before its own and
+// scans.  Three passes over the values (read; read and write) in place of the
+// six of a scan per block, a scan of the totals, an add per block and a copy
+// for the placement cursors: 131 -> 43 us for the 1.7e7 cells of 64 boxes of
+// 64^3, four launches -> two for a single box.
+constexpr int kScanPer = 16;
+constexpr int kScanTile = kBlock * kScanPer;
 
-struct k_scan_blocks {
-  static constexpr int kBounds = kBlock;
-  static __device__ __forceinline__ void run(int32_t *data, long n, int32_t *block_sums) {
-  __shared__ int32_t sh[kBlock];
-  long base = (long)blockIdx.x * kScanChunk + (long)threadIdx.x * kScanPer;
-  int32_t v[kScanPer];
-  int32_t tot = 0;
+// sum over the block, in every thread
+__device__ __forceinline__ int32_t block_total(int32_t v, int32_t *sh) {
 #pragma unroll
-  for (int e = 0; e < kScanPer; ++e) {
-    long q = base + e;
-    v[e] = q < n ? data[q] : 0;
-    tot += v[e];
-  }
-  sh[threadIdx.x] = tot;
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  const int w = (int)threadIdx.x >> 6;
   __syncthreads();
-  for (int off = 1; off < kBlock; off <<= 1) {
-    int32_t t = (int)threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-    __syncthreads();
-    sh[threadIdx.x] += t;
-    __syncthreads();
-  }
-  int32_t run = sh[threadIdx.x] - tot;  // exclusive prefix of this thread
-#pragma unroll
-  for (int e = 0; e < kScanPer; ++e) {
-    long q = base + e;
-    if (q < n) data[q] = run;
-    run += v[e];
-  }
-  if (threadIdx.x == kBlock - 1) block_sums[blockIdx.x] = sh[kBlock - 1];
+  if ((threadIdx.x & 63) == 0) sh[w] = v;
+  __syncthreads();
+  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
+
+struct k_scan_totals {
+  static constexpr int kBounds = kBlock;
+  static __device__ __forceinline__ void run(const int32_t *__restrict__ data, long n, int tiles, int32_t *totals) {
+    __shared__ int32_t sh[4];
+    const long lo = (long)blockIdx.x * tiles * kScanTile;
+    int32_t tot = 0;
+    for (int t = 0; t < tiles; ++t) {
+      int32_t v[kScanPer];
+#pragma unroll
+      for (int e = 0; e < kScanPer; ++e) {
+        const long q = lo + (long)t * kScanTile + e * kBlock + threadIdx.x;
+        v[e] = q < n ? data[q] : 0;
+      }
+#pragma unroll
+      for (int e = 0; e < kScanPer; ++e) tot += v[e];
+    }
+    tot = block_total(tot, sh);
+    if (threadIdx.x == 0) totals[blockIdx.x] = tot;
+  }
 };
 
-struct k_scan_add {
+struct k_scan_apply {
   static constexpr int kBounds = kBlock;
-  static __device__ __forceinline__ void run(int32_t *data, long n, const int32_t *offs) {
-  long q = (long)blockIdx.x * kScanChunk + threadIdx.x;
-  int32_t o = offs[blockIdx.x];
-  for (int e = 0; e < kScanPer; ++e, q += kBlock)
-    if (q < n) data[q] += o;
-}
+  static __device__ __forceinline__ void run(int32_t *data, long n, int tiles, const int32_t *__restrict__ totals) {
+    __shared__ int32_t sh[4], st[kScanTile + kScanTile / kScanPer];  // one spare slot every 16: no bank conflicts
+    const int tid = (int)threadIdx.x;
+    int32_t before = 0;
+    for (unsigned b = threadIdx.x; b < blockIdx.x; b += kBlock) before += totals[b];
+    before = block_total(before, sh);
+    const long lo = (long)blockIdx.x * tiles * kScanTile;
+    for (int t = 0; t < tiles; ++t) {
+      const long base = lo + (long)t * kScanTile;
+      int32_t v[kScanPer];
+#pragma unroll
+      for (int e = 0; e < kScanPer; ++e) {
+        const long q = base + e * kBlock + tid;
+        v[e] = q < n ? data[q] : 0;
+      }
+      __syncthreads();  // the last tile has been written out
+#pragma unroll
+      for (int e = 0; e < kScanPer; ++e) {
+        const int s = e * kBlock + tid;
+        st[s + s / kScanPer] = v[e];
+      }
+      __syncthreads();
+      // this thread's 16 consecutive values
+      int32_t own = 0;
+#pragma unroll
+      for (int e = 0; e < kScanPer; ++e) {
+        v[e] = st[tid * (kScanPer + 1) + e];
+        own += v[e];
+      }
+      int32_t inc = own;  // inclusive over the wave
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int32_t u = __shfl_up(inc, o, 64);
+        if ((tid & 63) >= o) inc += u;
+      }
+      if ((tid & 63) == 63) sh[tid >> 6] = inc;
+      __syncthreads();
+      int32_t run = before + inc - own;
+#pragma unroll
+      for (int w = 0; w < 3; ++w)
+        if (w < (tid >> 6)) run += sh[w];
+      before += (sh[0] + sh[1]) + (sh[2] + sh[3]);
+#pragma unroll
+      for (int e = 0; e < kScanPer; ++e) {
+        st[tid * (kScanPer + 1) + e] = run;
+        run += v[e];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < kScanPer; ++e) {
+        const int s = e * kBlock + tid;
+        if (base + s < n) data[base + s] = st[s + s / kScanPer];
+      }
+    }
+  }
 };
 
 // ---- deposits ----
@@ -841,38 +888,27 @@ void launch_iota(tpx_ctx *c, int32_t *p, int64_t n) {
 }
 
 void launch_exclusive_scan(tpx_ctx *c, int32_t *data, int64_t n) {
-  // recursive three-phase scan; block sums of level l live in scan_tmp
-  std::vector<std::pair<int32_t *, long>> levels;
-  int32_t *cur = data;
-  long len = n;
-  int32_t *tmp = c->scan_tmp;
-  while (true) {
-    long nb = (len + kScanChunk - 1) / kScanChunk;
-    tpx_launch<k_scan_blocks>((unsigned)nb, kBlock, 0, c->stream, cur, len, tmp);
-    TPX_LAUNCH_CHECK();
-    levels.push_back({cur, len});
-    if (nb == 1) break;
-    cur = tmp;
-    len = nb;
-    tmp = tmp + nb;
-  }
-  for (int l = (int)levels.size() - 2; l >= 0; --l) {
-    long len_l = levels[l].second;
-    long nb = (len_l + kScanChunk - 1) / kScanChunk;
-    tpx_launch<k_scan_add>((unsigned)nb, kBlock, 0, c->stream, levels[l].first, len_l, levels[l + 1].first);
-    TPX_LAUNCH_CHECK();
-  }
+  // at most 8192 blocks: each reads the totals of all before it
+  int tiles = 1;
+  while ((n + (int64_t)tiles * kScanTile - 1) / ((int64_t)tiles * kScanTile) > 8192) tiles *= 2;
+  const unsigned nb = (unsigned)((n + (int64_t)tiles * kScanTile - 1) / ((int64_t)tiles * kScanTile));
+  tpx_launch<k_scan_totals>(nb, kBlock, 0, c->stream, (const int32_t *)data, (long)n, tiles, c->scan_tmp);
+  TPX_LAUNCH_CHECK();
+  tpx_launch<k_scan_apply>(nb, kBlock, 0, c->stream, data, (long)n, tiles, (const int32_t *)c->scan_tmp);
+  TPX_LAUNCH_CHECK();
 }
 
 // Stable bins of the particles by key (one int per particle): perm (sorted
 // position -> particle), inv (particle -> sorted position), start (CSR).
-// On entry `start` holds the per-cell counts (start[n_cell] = 0).
+// On entry start[c + 1] holds the count of cell c and start[0] is 0.  The scan
+// leaves each cell's first slot at start[c + 1], the placement moves it on to
+// one past its last, which is the first slot of cell c + 1: start is then the
+// CSR, with no cursors of its own.
 static void bin_particles(tpx_ctx *c, const int32_t *key, int32_t *perm, int32_t *inv, int32_t *start) {
   Particles &pt = c->pt;
   long n = pt.n, nc = c->g.n;
-  launch_exclusive_scan(c, start, nc + 1);
-  tpx_launch<k_copy_i>(grid1d(nc + 1, kBlock), kBlock, 0, c->stream, pt.cursor, start, nc + 1);
-  tpx_launch<k_place>(grid1d(n, kBlock), kBlock, 0, c->stream, key, pt.cursor, perm, n);
+  launch_exclusive_scan(c, start + 1, nc);
+  tpx_launch<k_place>(grid1d(n, kBlock), kBlock, 0, c->stream, key, start + 1, perm, n);
   tpx_launch<k_fixup>(grid1d(nc, kBlock), kBlock, 0, c->stream, start, perm, inv, nc);
   TPX_LAUNCH_CHECK();
 }
@@ -912,7 +948,7 @@ void launch_particle_advance(tpx_ctx *c, const Coef &k, const double *const ru_i
   a.contrib = c->p.twc ? pt.contrib : nullptr;
   a.cstride = pt.cap;
   a.inv_int = pt.inv_int;
-  a.cnt = count_new ? pt.start_new : nullptr;
+  a.cnt = count_new ? pt.start_new + 1 : nullptr;
   a.key = pt.key;
   a.n = pt.n;
   a.int_is_base = pt.int_is_base || si == sb;
@@ -1093,7 +1129,7 @@ void launch_sort_stage(tpx_ctx *c, int stage, bool into_int) {
   int32_t *start = into_int ? pt.start_int : pt.start_new;
   timing_begin(c, TPX_K_SORT);
   zero_counts(c, start);
-  tpx_launch<k_keys>(grid1d(pt.n, kBlock), kBlock, 0, c->stream, c->g, pt.q[0][s], pt.q[1][s], pt.q[2][s], pt.key, start,
+  tpx_launch<k_keys>(grid1d(pt.n, kBlock), kBlock, 0, c->stream, c->g, pt.q[0][s], pt.q[1][s], pt.q[2][s], pt.key, start + 1,
                                                          pt.n);
   TPX_LAUNCH_CHECK();
   bin_particles(c, pt.key, into_int ? pt.perm_int : pt.perm_new, into_int ? pt.inv_int : pt.inv_new, start);

@@ -720,7 +720,7 @@ void release(tpx_ctx *c) {
   Particles &pt = c->pt;
   for (auto &q : pt.q) for (auto &p : q) f(p);
   f(pt.rhs_t); f(pt.tau); f(pt.eps); f(pt.flag); f(pt.contrib); f(pt.key);
-  f(pt.perm_int); f(pt.perm_new); f(pt.start_int); f(pt.start_new); f(pt.cursor);
+  f(pt.perm_int); f(pt.perm_new); f(pt.start_int); f(pt.start_new);
   f(pt.inv_int); f(pt.inv_new);
   for (auto &p : pt.spare) f(p);
   f(pt.itmp);
@@ -844,7 +844,7 @@ int tpx_create(const tpx_params *p, int64_t np_capacity, tpx_ctx **out) {
     // one partial per 256-cell block or per x-row, whichever is more
     c->n_partials = std::max((long)grid1d(g.n, 256), (long)g.ny * g.nz) + 1024;
     dalloc(&c->partials, 3 * (size_t)c->n_partials);
-    ialloc(&c->scan_tmp, (size_t)(g.n / 2048 + 1024));
+    ialloc(&c->scan_tmp, 8192);  // block totals of a scan
     // one pinned block (each allocation costs some 0.3 ms here and as much
     // again to free): the scalars' mirror, the solves' loop state on a line of
     // its own, and the first copying thread's chunks
@@ -877,7 +877,7 @@ int tpx_create(const tpx_params *p, int64_t np_capacity, tpx_ctx **out) {
     ialloc(&pt.key, cap);
     ialloc(&pt.perm_int, cap); ialloc(&pt.perm_new, cap);
     ialloc(&pt.inv_int, cap); ialloc(&pt.inv_new, cap);
-    ialloc(&pt.start_int, n + 1); ialloc(&pt.start_new, n + 1); ialloc(&pt.cursor, n + 1);
+    ialloc(&pt.start_int, n + 1); ialloc(&pt.start_new, n + 1);
     hip_check(hipMemset(pt.start_int, 0, sizeof(int32_t) * (n + 1)), "hipMemset");
     hip_check(hipMemset(pt.rhs_t, 0, sizeof(double) * (cap ? cap : 1)), "hipMemset");
     hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");

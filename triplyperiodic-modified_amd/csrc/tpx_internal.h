@@ -103,7 +103,6 @@ struct Particles {
   int32_t *perm_int = nullptr, *perm_new = nullptr;     // sorted position -> particle
   int32_t *inv_int = nullptr, *inv_new = nullptr;       // particle -> sorted position
   int32_t *start_int = nullptr, *start_new = nullptr;   // CSR over cells (n_cell+1)
-  int32_t *cursor = nullptr;      // placement cursors over cells (n_cell+1)
   bool new_counted = false;       // the last advance counted x_new into start_new
   bool has_tau = false, has_eps = false;
   // spare arrays the step-end permutation writes into (rhs_t, tau, eps, flag)
@@ -335,7 +334,7 @@ struct tpx_ctx {
   long st_stride = 0;
   long n_partials = 0;
   double *h_scal = nullptr;       // pinned host mirror of scal
-  int32_t *scan_tmp = nullptr;    // scan block sums
+  int32_t *scan_tmp = nullptr;    // scan block totals
   tpx::Particles pt;
   tpx::Timing tm;
   tpx::HostStage stage;
@@ -419,12 +418,12 @@ void launch_particle_permute(tpx_ctx *c);
 void launch_sort_stage(tpx_ctx *c, int stage, bool into_int);
 void launch_iota(tpx_ctx *c, int32_t *p, int64_t n);
 // Deterministic cell bins of the particles' keys (the particle path's
-// binning): start (cells + 1) holds each cell's count on entry and its first
-// slot on return, perm the particles in cell order (each cell's by index),
+// binning): start (cells + 1) holds 0 and each cell's count on entry, each
+// cell's first slot and the total on return, perm the particles in cell order (each cell's by index),
 // inv its inverse.  launch_zero_counts clears the cells + 1 counts.
 void launch_bin_by_key(tpx_ctx *c, const int32_t *key, int32_t *perm, int32_t *inv, int32_t *start);
 void launch_zero_counts(tpx_ctx *c, int32_t *cnt);
-void launch_exclusive_scan(tpx_ctx *c, int32_t *data, int64_t n);  // in place, n+1 output
+void launch_exclusive_scan(tpx_ctx *c, int32_t *data, int64_t n);  // in place
 
 // k_adjoint.hip
 void adjoint_tape_substep(tpx_ctx *c, int rk, const double *const ru_int[3], const double *rho_int);
