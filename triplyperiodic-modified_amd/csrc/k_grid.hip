@@ -73,6 +73,18 @@ __device__ __forceinline__ double Uface(const Ix &ix, const double *__restrict__
   return ru[p] / ((rho[p] + rho[q]) * 0.5);
 }
 
+// grid::Update_P0 (grid.cpp:816-830) on the device scalars
+__device__ __forceinline__ void update_p0(const Coef &kc, double *scal, double ncell) {
+  const double c_np1 = kc.dt * kc.post, c_new = kc.dt * kc.pre;
+  double met = scal[SC_SUM_Q] / ncell;
+  scal[SC_MET] = met;
+  double dP0 = kc.cooling ? 0.0 : -kc.R / kc.cv * met / kc.Vcell;
+  scal[SC_DP0_DT] = dP0;
+  scal[SC_P0_NP1] += c_np1 * dP0;
+  if (kc.rk != 3) scal[SC_P0_NEW] = scal[SC_P0] + c_new * dP0;
+  else scal[SC_P0_NEW] = scal[SC_P0_NP1];
+}
+
 struct RU3 { const double *__restrict__ a[3]; };
 
 // div_F2C(U) at cell centre (i,j,k) (tensor0.cpp:249-256)
@@ -95,8 +107,10 @@ struct RhsArgs {
   const double *rho_np1_in;
   double *rho_np1;
   double *rho_new;
+  double *p0_scal = nullptr;  // non-null: one thread of the launch also does Update_P0
   double c_np1, c_new, c_rho_np1, c_rho_new;
   __device__ void to_global() {
+    p0_scal = gptr(p0_scal);
     for (int c = 0; c < 3; ++c) {
       ru_int.a[c] = gptr(ru_int.a[c]);
       ru_base[c] = gptr(ru_base[c]);
@@ -246,8 +260,12 @@ struct ProjArgs {
   double *nw[3];
   double *partials;
   long npart;
+  double *scal = nullptr;    // non-null: P0_int = P0_new too (grid.cpp:898)
+  int32_t *zero = nullptr;   // non-null: cleared from zero[1] on, one value a cell
   double c_np1, c_new;
   __device__ void to_global() {
+    scal = gptr(scal);
+    zero = gptr(zero);
     P = gptr(P);
     for (int q = 0; q < 3; ++q) np1[q] = gptr(np1[q]);
     for (int q = 0; q < 3; ++q) nw[q] = gptr(nw[q]);
@@ -267,7 +285,9 @@ struct k_project {
   bool ok = cell_of(g, i, j, k, c);
   Ix ix = make_ix(g);
   double s[3] = {0, 0, 0};
+  if (a.scal && blockIdx.x == 0 && threadIdx.x == 0) a.scal[SC_P0_INT] = a.scal[SC_P0_NEW];
   if (ok) {
+    if (a.zero) a.zero[c + 1] = 0;
     const double *__restrict__ P = a.P;
     double pc = P[c];
     double gr[3] = {(pc - P[ix(i - 1, j, k)]) * g.idx, (pc - P[ix(i, j - 1, k)]) * g.idy,
@@ -291,17 +311,35 @@ struct k_project {
 }
 };
 
-// tensor0::make_mean_U0 (tensor0.cpp:386-396): out = (in - mean) + a
+struct ShiftArgs {
+  const double *in[3];
+  double *out[3];
+  double a[3];
+  double *scal;
+  double ncell;
+  int p0;  // nonzero: P0 = P0_np1 too (grid.cpp:602)
+  __device__ void to_global() {
+    for (int d = 0; d < 3; ++d) {
+      in[d] = gptr(in[d]);
+      out[d] = gptr(out[d]);
+    }
+    scal = gptr(scal);
+  }
+};
+
+// tensor1::make_mean_U0 (tensor1.cpp:406-411, tensor0.cpp:386-396): out = (in - mean) + a
 struct k_shift_mean {
   static constexpr int kBounds = kBlock;
-  static __device__ __forceinline__ void run(long n, const double *__restrict__ in,
-                                                       double *__restrict__ out, const double *scal,
-                                                       int slot, double ncell, double a) {
-  long c = (long)blockIdx.x * block_dim_x() + threadIdx.x;
-  if (c >= n) return;
-  double mean = scal[slot] / ncell;  // mean() = sum()/size_tot()
-  out[c] = (in[c] - mean) + a;
-}
+  static __device__ __forceinline__ void run(long n, const ShiftArgs &s) {
+    long c = (long)blockIdx.x * block_dim_x() + threadIdx.x;
+    if (s.p0 && c == 0) s.scal[SC_P0] = s.scal[SC_P0_NP1];
+    if (c >= n) return;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      double mean = s.scal[SC_MEAN_RU0 + d] / s.ncell;  // mean() = sum()/size_tot()
+      s.out[d][c] = (s.in[d][c] - mean) + s.a[d];
+    }
+  }
 };
 
 // generic reduction of one field into per-block partials
@@ -319,15 +357,17 @@ struct k_reduce {
 }
 };
 
-// sum (OP 0) or max (OP 1) of nparts partials into scal[slot], fixed order:
+// sum (OP 0) or max (OP 1) of nparts partials into scal[slot] (block b: of the
+// b-th nparts partials into scal[slot + b]), fixed order:
 // thread t combines partials t, t + 1024, t + 2048, ... (coalesced reads,
 // four independent accumulators), then the block tree
 template <int OP>
 struct k_finish {
   static constexpr int kBounds = 1024;
-  static __device__ __forceinline__ void run(const double *__restrict__ partials, long nparts,
+  static __device__ __forceinline__ void run(const double *__restrict__ all, long nparts,
                                                  double *scal, int slot) {
   __shared__ double sh[1024];
+  const double *__restrict__ partials = all + blockIdx.x * nparts;
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
   long q = threadIdx.x;
   for (; q + 3 * 1024 < nparts; q += 4 * 1024) {
@@ -340,23 +380,15 @@ struct k_finish {
   for (int u = 0; q < nparts; q += 1024, ++u) acc[u] = OP == 0 ? acc[u] + partials[q] : fmax(acc[u], partials[q]);
   double v = OP == 0 ? (acc[0] + acc[1]) + (acc[2] + acc[3]) : fmax(fmax(acc[0], acc[1]), fmax(acc[2], acc[3]));
   double s = OP == 0 ? block_sum(v, sh) : block_max(v, sh);
-  if (threadIdx.x == 0) scal[slot] = s;
+  if (threadIdx.x == 0) scal[slot + blockIdx.x] = s;
 }
 };
 
-// grid::Update_P0 (grid.cpp:816-830) on the device scalars
 struct k_update_p0 {
   static constexpr int kBounds = 1024;
-  static __device__ __forceinline__ void run(const Coef &kc, double *scal, double ncell, double c_np1, double c_new) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  double met = scal[SC_SUM_Q] / ncell;
-  scal[SC_MET] = met;
-  double dP0 = kc.cooling ? 0.0 : -kc.R / kc.cv * met / kc.Vcell;
-  scal[SC_DP0_DT] = dP0;
-  scal[SC_P0_NP1] += c_np1 * dP0;
-  if (kc.rk != 3) scal[SC_P0_NEW] = scal[SC_P0] + c_new * dP0;
-  else scal[SC_P0_NEW] = scal[SC_P0_NP1];
-}
+  static __device__ __forceinline__ void run(const Coef &kc, double *scal, double ncell) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) update_p0(kc, scal, ncell);
+  }
 };
 
 struct k_scalar_copy {
@@ -408,8 +440,9 @@ void launch_rhs_ru(tpx_ctx *c, const Coef &k, bool with_rho, const double *const
                    const double *rho_int, const double *const ru_base[3],
                    const double *const ru_np1_in[3], const double *const S[3],
                    double *const ru_np1[3], double *const ru_new[3], const double *rho_base,
-                   const double *rho_np1_in, double *rho_np1, double *rho_new) {
+                   const double *rho_np1_in, double *rho_np1, double *rho_new, bool with_p0) {
   RhsArgs a{};
+  a.p0_scal = with_p0 ? c->scal : nullptr;
   for (int d = 0; d < 3; ++d) {
     a.ru_int.a[d] = ru_int[d];
     a.ru_base[d] = ru_base[d];
@@ -570,8 +603,10 @@ void launch_div_rhs(tpx_ctx *c, const Coef &k, int mode, const double *const ru_
 }
 
 void launch_project(tpx_ctx *c, const Coef &k, const double *P, double *const ru_np1[3],
-                    double *const ru_new[3], bool copy_np1_to_new, bool want_sums) {
+                    double *const ru_new[3], bool copy_np1_to_new, bool want_sums, bool advance_p0, int32_t *zero) {
   ProjArgs a{};
+  a.scal = advance_p0 ? c->scal : nullptr;
+  a.zero = zero;
   a.P = P;
   for (int d = 0; d < 3; ++d) { a.np1[d] = ru_np1[d]; a.nw[d] = ru_new[d]; }
   a.partials = c->partials;
@@ -586,19 +621,24 @@ void launch_project(tpx_ctx *c, const Coef &k, const double *P, double *const ru
   timing_end(c, TPX_K_PROJECT);
   if (copy_np1_to_new && want_sums) {
     timing_begin(c, TPX_K_OTHER);
-    for (int d = 0; d < 3; ++d)
-      tpx_launch<k_finish<0>>(1, 1024, 0, c->stream, c->partials + (long)d * nb, nb, c->scal, SC_MEAN_RU0 + d);
+    tpx_launch<k_finish<0>>(3, 1024, 0, c->stream, (const double *)c->partials, (long)nb, c->scal, (int)SC_MEAN_RU0);
     TPX_LAUNCH_CHECK();
     timing_end(c, TPX_K_OTHER);
   }
 }
 
-void launch_shift_mean(tpx_ctx *c, const double *const in[3], double *const out[3],
-                       const double a[3]) {
+void launch_shift_mean(tpx_ctx *c, const double *const in[3], double *const out[3], const double a[3], bool advance_p0) {
+  ShiftArgs s{};
+  for (int d = 0; d < 3; ++d) {
+    s.in[d] = in[d];
+    s.out[d] = out[d];
+    s.a[d] = a[d];
+  }
+  s.scal = c->scal;
+  s.ncell = (double)c->g.n;
+  s.p0 = advance_p0;
   timing_begin(c, TPX_K_OTHER);
-  for (int d = 0; d < 3; ++d)
-    tpx_launch<k_shift_mean>(cells_grid(c), kBlock, 0, c->stream, c->g.n, in[d], out[d], c->scal,
-                                                         SC_MEAN_RU0 + d, (double)c->g.n, a[d]);
+  tpx_launch<k_shift_mean>(cells_grid(c), kBlock, 0, c->stream, c->g.n, s);
   TPX_LAUNCH_CHECK();
   timing_end(c, TPX_K_OTHER);
 }
@@ -655,7 +695,7 @@ void launch_passive_scalar_source_sum(tpx_ctx *c) {
 
 void launch_update_p0(tpx_ctx *c, const Coef &k) {
   timing_begin(c, TPX_K_OTHER);
-  tpx_launch<k_update_p0>(1, 64, 0, c->stream, k, c->scal, (double)c->g.n, k.dt * k.post, k.dt * k.pre);
+  tpx_launch<k_update_p0>(1, 64, 0, c->stream, k, c->scal, (double)c->g.n);
   TPX_LAUNCH_CHECK();
   timing_end(c, TPX_K_OTHER);
 }

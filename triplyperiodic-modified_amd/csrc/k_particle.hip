@@ -835,7 +835,8 @@ struct k_concentration {
 };
 
 struct PermArgs {
-  const int32_t *perm;       // sorted position -> particle
+  int32_t *perm;             // sorted position -> particle; the identity on return
+  int32_t *inv;              // its inverse, likewise
   const double *src[7];
   double *dst[7];
   const double *s1[3];
@@ -845,6 +846,7 @@ struct PermArgs {
   long n;
   __device__ void to_global() {
     perm = gptr(perm);
+    inv = gptr(inv);
     for (int q = 0; q < 7; ++q) src[q] = gptr(src[q]);
     for (int q = 0; q < 7; ++q) dst[q] = gptr(dst[q]);
     for (int q = 0; q < 3; ++q) s1[q] = gptr(s1[q]);
@@ -869,6 +871,8 @@ struct k_permute {
   for (int d = 0; d < 3; ++d)
     if (a.s1[d]) a.d1[d][q] = a.s1[d][s];
   a.flag_d[q] = a.flag_s[s];
+  a.perm[q] = (int32_t)q;
+  a.inv[q] = (int32_t)q;
 }
 };
 
@@ -965,7 +969,8 @@ void launch_particle_advance(tpx_ctx *c, const Coef &k, const double *const ru_i
   a.rk3 = k.rk == 3;
   if (count_new) {
     timing_begin(c, TPX_K_SORT);
-    zero_counts(c, pt.start_new);
+    if (!pt.new_zeroed) zero_counts(c, pt.start_new);
+    pt.new_zeroed = false;
     timing_end(c, TPX_K_SORT);
   }
   timing_begin(c, TPX_K_ADVANCE);
@@ -1128,6 +1133,7 @@ void launch_sort_stage(tpx_ctx *c, int stage, bool into_int) {
   int s = stage == TPX_BASE ? pt.st_base : stage == TPX_INT ? pt.int_buf() : stage == TPX_NEW ? pt.st_new : pt.st_np1;
   int32_t *start = into_int ? pt.start_int : pt.start_new;
   timing_begin(c, TPX_K_SORT);
+  if (!into_int) pt.new_zeroed = false;
   zero_counts(c, start);
   tpx_launch<k_keys>(grid1d(pt.n, kBlock), kBlock, 0, c->stream, c->g, pt.q[0][s], pt.q[1][s], pt.q[2][s], pt.key, start + 1,
                                                          pt.n);
@@ -1206,6 +1212,7 @@ void launch_particle_permute(tpx_ctx *c) {
   int dst = pt.st_np1;  // np1 is stale (np1_is_base)
   PermArgs a{};
   a.perm = pt.perm_int;
+  a.inv = pt.inv_int;
   for (int q = 0; q < 7; ++q) {
     a.src[q] = pt.q[q][sb];
     a.dst[q] = pt.q[q][dst];
@@ -1236,8 +1243,6 @@ void launch_particle_permute(tpx_ctx *c) {
       if (b != used[0] && b != used[1] && b != used[2]) pt.st_int = b;
   }
   pt.int_is_base = true;
-  launch_iota(c, pt.perm_int, pt.n);
-  launch_iota(c, pt.inv_int, pt.n);
   timing_end(c, TPX_K_SORT);
   check(hipGetLastError());
 }

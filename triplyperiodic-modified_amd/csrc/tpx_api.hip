@@ -392,7 +392,9 @@ void do_update_passive_scalar(tpx_ctx *c, int rk) {
   launch_passive_scalar(c, k, ri, c->rho[c->rho_int]);
 }
 
-void do_update_ru_wop(tpx_ctx *c, int rk, bool with_rho) {
+// with_p0: Update_P0 rides in the same launch (nothing before it in the fused
+// substep reads its results)
+void do_update_ru_wop(tpx_ctx *c, int rk, bool with_rho, bool with_p0 = false) {
   Coef k = coef(c, rk);
   int np1_in = ru_np1_read(c);
   int rho_np1_in = rho_np1_read(c);
@@ -409,7 +411,7 @@ void do_update_ru_wop(tpx_ctx *c, int rk, bool with_rho) {
   const double *S[3] = {c->S[0], c->S[1], c->S[2]};
   launch_rhs_ru(c, k, with_rho, ri, c->rho[c->rho_int], rb, rn, has_s ? S : nullptr, on, ow,
                 c->rho[c->rho_base], c->rho[rho_np1_in],
-                with_rho ? c->rho[c->rho_np1] : nullptr, with_rho ? c->rho[c->rho_new] : nullptr);
+                with_rho ? c->rho[c->rho_np1] : nullptr, with_rho ? c->rho[c->rho_new] : nullptr, with_p0);
 }
 
 // Waits until the running solve has stopped or finished `want` iterations;
@@ -540,20 +542,22 @@ void do_passive_vector(tpx_ctx *c, int rk) {
   do_update_rv_wq(c, rk);
 }
 
-void do_update_ru_wp(tpx_ctx *c, int rk, bool want_sums) {
+// advance_p0: TimeAdvance_RK4's P0_int = P0_new rides in the same launch; zero:
+// per-cell counts cleared in it
+void do_update_ru_wp(tpx_ctx *c, int rk, bool want_sums, bool advance_p0 = false, int32_t *zero = nullptr) {
   Coef k = coef(c, rk);
   double *on[3], *ow[3];
   ru_wptrs(c, c->ru_np1, on);
   ru_wptrs(c, c->ru_new, ow);
-  launch_project(c, k, c->P, on, ow, rk == 3, want_sums);
+  launch_project(c, k, c->P, on, ow, rk == 3, want_sums, advance_p0, zero);
 }
 
-void do_time_advance_rk4(tpx_ctx *c) {
+void do_time_advance_rk4(tpx_ctx *c, bool p0_done = false, bool int_zeroed = false) {
   c->rho_int = c->rho_new;
   c->ru_int = c->ru_new;
   c->rho_new = -1;
   c->ru_new = -1;
-  launch_scalar_copy(c, SC_P0_INT, SC_P0_NEW);
+  if (!p0_done) launch_scalar_copy(c, SC_P0_INT, SC_P0_NEW);
   if (c->ps[0]) std::swap(c->ps_int, c->ps_new);  // Passive_Scalar_int = Passive_Scalar_new (grid.cpp:897)
   if (c->Qv) std::swap(c->rv_int, c->rv_new);     // RV_int = RV_new (grid.cpp:894)
   Particles &pt = c->pt;
@@ -562,9 +566,11 @@ void do_time_advance_rk4(tpx_ctx *c) {
   std::swap(pt.perm_int, pt.perm_new);
   std::swap(pt.inv_int, pt.inv_new);
   std::swap(pt.start_int, pt.start_new);
+  pt.new_zeroed = int_zeroed;
 }
 
-void do_make_mean_u0(tpx_ctx *c, const double a[3], bool sums_ready) {
+// advance_p0: TimeAdvance's P0 = P0_np1 rides in the same launch
+void do_make_mean_u0(tpx_ctx *c, const double a[3], bool sums_ready, bool advance_p0 = false) {
   int src = ru_np1_read(c);
   if (!sums_ready)
     for (int d = 0; d < 3; ++d) launch_reduce(c, c->ru[src][d], 0, SC_MEAN_RU0 + d);
@@ -573,17 +579,17 @@ void do_make_mean_u0(tpx_ctx *c, const double a[3], bool sums_ready) {
   double *out[3];
   ru_ptrs(c, src, in);
   ru_wptrs(c, dst, out);
-  launch_shift_mean(c, in, out, a);
+  launch_shift_mean(c, in, out, a, advance_p0);
   c->ru_np1 = dst;
   c->ru_np1_is_base = false;
 }
 
-void do_time_advance(tpx_ctx *c) {
+void do_time_advance(tpx_ctx *c, bool p0_done = false) {
   c->rho_base = rho_np1_read(c);
   c->rho_np1_is_base = true;
   c->ru_base = ru_np1_read(c);
   c->ru_np1_is_base = true;
-  launch_scalar_copy(c, SC_P0, SC_P0_NP1);
+  if (!p0_done) launch_scalar_copy(c, SC_P0, SC_P0_NP1);
   if (c->ps[0]) launch_copy(c, c->ps[c->ps_base], c->ps[c->ps_np1], c->g.n);  // grid.cpp:598
   if (c->Qv)  // RV = RV_np1 (grid.cpp:600)
     for (int d = 0; d < 3; ++d) launch_copy(c, c->rv[c->rv_base][d], c->rv[c->rv_np1][d], c->g.n);
@@ -615,7 +621,6 @@ void do_params_update(tpx_ctx *c) {
 // part before the Poisson solve:
 void fused_substep_pre(tpx_ctx *c, int rk) {
   Coef k = coef(c, rk);
-  launch_update_p0(c, k);
   Particles &pt = c->pt;
   bool parts = pt.n > 0;
   bool rebin = parts && (c->p.twc || heat_active(c));
@@ -633,7 +638,7 @@ void fused_substep_pre(tpx_ctx *c, int rk) {
   }
   if (c->p.solve_for_scalar) do_update_passive_scalar(c, rk);  // simulation.cpp:65
   if (c->p.solve_for_vector) do_passive_vector(c, rk);          // simulation.cpp:66-71
-  do_update_ru_wop(c, rk, true);
+  do_update_ru_wop(c, rk, true, true);
   if (rebin) {
     launch_sort_new(c);
     c->binned_this_step = true;
@@ -655,8 +660,12 @@ void fused_substep_pre(tpx_ctx *c, int rk) {
 }
 
 void fused_substep_post(tpx_ctx *c, int rk) {
-  do_update_ru_wp(c, rk, rk == 3);
-  do_time_advance_rk4(c);
+  // the bins of x_int have served their substep: cleared here, they are the
+  // counts of the next one's x_new
+  Particles &pt = c->pt;
+  const bool rebin = pt.n > 0 && (c->p.twc || heat_active(c));
+  do_update_ru_wp(c, rk, rk == 3, true, rebin ? pt.start_int : nullptr);
+  do_time_advance_rk4(c, true, rebin);
 }
 
 void fused_substep(tpx_ctx *c, int rk) {
@@ -668,8 +677,8 @@ void fused_substep(tpx_ctx *c, int rk) {
 // the end of a step after its four substeps (simulation.cpp:80-82)
 void step_end(tpx_ctx *c) {
   const double a[3] = {c->p.u0 * c->p.rho0, c->p.v0 * c->p.rho0, c->p.w0 * c->p.rho0};
-  do_make_mean_u0(c, a, true);
-  do_time_advance(c);
+  do_make_mean_u0(c, a, true, true);
+  do_time_advance(c, true);
 }
 
 // frees every array of a recorded adjoint run
@@ -1718,8 +1727,6 @@ void gas_substeps(tpx_ctx *c, int s, GasSubstep sub[4], bool segment) {
       g.Q = t.qt + (long)q * n;
       g.q_sum = t.qs + q;
       g.p0n = t.p0t + q + 1;
-    } else {
-      launch_update_p0(c, k);
     }
     {
       // two-way coupling: the momentum update reads the recorded drag deposit
@@ -1729,7 +1736,7 @@ void gas_substeps(tpx_ctx *c, int s, GasSubstep sub[4], bool segment) {
       if (t.S)
         for (int d = 0; d < 3; ++d) c->S[d] = t.S + (((long)s * 4 + rk) * 3 + d) * n;
       try {
-        do_update_ru_wop(c, rk, true);
+        do_update_ru_wop(c, rk, true, !t.heat);
       } catch (...) {
         for (int d = 0; d < 3; ++d) c->S[d] = keep[d];
         throw;
@@ -1773,21 +1780,19 @@ void gas_substeps(tpx_ctx *c, int s, GasSubstep sub[4], bool segment) {
       c->iter_ctl.first = 0;
     }
     launch_copy(c, t.iters_seen + (long)s * 4 + rk, c->scal + SC_ITERS, 1);
-    do_update_ru_wp(c, rk, rk == 3);
+    do_update_ru_wp(c, rk, rk == 3, true);
     c->rho_int = c->rho_new;  // the gas half of TimeAdvance_RK4
     c->ru_int = c->ru_new;
     c->rho_new = -1;
     c->ru_new = -1;
-    launch_scalar_copy(c, SC_P0_INT, SC_P0_NEW);
   }
   if (segment) t.pnext = used;
   const double a[3] = {c->p.u0 * c->p.rho0, c->p.v0 * c->p.rho0, c->p.w0 * c->p.rho0};
-  do_make_mean_u0(c, a, true);
+  do_make_mean_u0(c, a, true, true);
   c->rho_base = rho_np1_read(c);  // the gas half of TimeAdvance
   c->rho_np1_is_base = true;
   c->ru_base = ru_np1_read(c);
   c->ru_np1_is_base = true;
-  launch_scalar_copy(c, SC_P0, SC_P0_NP1);
 }
 
 // Recomputes step s of the recorded run from its start on the tape (RU and P
@@ -2021,6 +2026,11 @@ int tpx_batch_step(tpx_batch *b, int nsteps) {
       if (c->tile.active) throw std::logic_error("a box is still tuning its tile shapes: step it alone first");
       sync(c);
     }
+    // every box must launch the same kernels: all clear their counts anew
+    // unless all are known to be clear
+    bool zeroed = true;
+    for (tpx_ctx *c : b->ctx) zeroed = zeroed && c->pt.new_zeroed;
+    for (tpx_ctx *c : b->ctx) c->pt.new_zeroed = zeroed;
     for (int s = 0; s < nsteps; ++s) {
       for (tpx_ctx *c : b->ctx) do_params_update(c);
       for (int rk = 0; rk < 4; ++rk) {

@@ -104,6 +104,7 @@ struct Particles {
   int32_t *inv_int = nullptr, *inv_new = nullptr;       // particle -> sorted position
   int32_t *start_int = nullptr, *start_new = nullptr;   // CSR over cells (n_cell+1)
   bool new_counted = false;       // the last advance counted x_new into start_new
+  bool new_zeroed = false;        // start_new is all zero: the next advance can count into it
   bool has_tau = false, has_eps = false;
   // spare arrays the step-end permutation writes into (rhs_t, tau, eps, flag)
   double *spare[3] = {};
@@ -353,15 +354,15 @@ void launch_rhs_ru(tpx_ctx *c, const Coef &k, bool with_rho, const double *const
                    const double *const ru_np1_in[3], const double *const S[3],
                    double *const ru_np1[3], double *const ru_new[3],
                    const double *rho_base, const double *rho_np1_in, double *rho_np1,
-                   double *rho_new);
+                   double *rho_new, bool with_p0);
 // mode 0: fused (write rhs + partial sums); 1: write divergence only;
 // 2: read divergence, write rhs + partial sums
 void launch_div_rhs(tpx_ctx *c, const Coef &k, int mode, const double *const ru_new[3],
                     const double *rho_new, const double *Q, double *divergence, double *rhs);
 void launch_project(tpx_ctx *c, const Coef &k, const double *P, double *const ru_np1[3],
-                    double *const ru_new[3], bool copy_np1_to_new, bool want_sums);
-void launch_shift_mean(tpx_ctx *c, const double *const in[3], double *const out[3],
-                       const double a[3]);
+                    double *const ru_new[3], bool copy_np1_to_new, bool want_sums, bool advance_p0, int32_t *zero);
+void launch_shift_mean(tpx_ctx *c, const double *const in[3], double *const out[3], const double a[3],
+                       bool advance_p0);
 void launch_reduce(tpx_ctx *c, const double *f, int op, int slot);  // op 0 sum, 1 max|.|, 2 sum of squares
 void launch_finish_sum(tpx_ctx *c, int nparts, int part_offset, int slot);
 void launch_update_p0(tpx_ctx *c, const Coef &k);
