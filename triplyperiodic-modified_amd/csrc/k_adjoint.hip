@@ -275,6 +275,24 @@ struct k_adj_gather_pull {
 
 // Keys and counts of the bins of positions (x, y, z rows of Y): the gather's
 // cell (floor), or with cic set the cloud-in-cell base corner (round - 1)
+struct k_sum3 {
+  static constexpr int kBounds = kBlock;
+  static __device__ __forceinline__ void run(const double *__restrict__ a, const double *__restrict__ b,
+                                             const double *__restrict__ d, double *__restrict__ out, long n) {
+    const long q = (long)blockIdx.x * block_dim_x() + threadIdx.x;
+    if (q < n) out[q] = (a[q] + b[q]) + d[q];
+  }
+};
+
+struct k_take {
+  static constexpr int kBounds = kBlock;
+  static __device__ __forceinline__ void run(const double *__restrict__ src, const int32_t *__restrict__ idx,
+                                             double *__restrict__ out, long n) {
+    const long q = (long)blockIdx.x * block_dim_x() + threadIdx.x;
+    if (q < n) out[q] = src[idx[q]];
+  }
+};
+
 struct k_adj_bin_keys {
   static constexpr int kBounds = kBlock;
   static __device__ __forceinline__ void run(const Geo &g, const double *Y, int cic, int32_t *key, int32_t *cnt,
@@ -691,6 +709,16 @@ StepArgs step_args(tpx_ctx *c, int step, const double *const yin[7], double *con
 }  // namespace
 
 // copies this substep's RU_int and Rho_int into the tape
+void launch_sum3(tpx_ctx *c, const double *a, const double *b, const double *d, double *out, long n) {
+  tpx_launch<k_sum3>(grid1(n), kBlock, 0, c->stream, a, b, d, out, n);
+  TPX_LAUNCH_CHECK();
+}
+
+void launch_take(tpx_ctx *c, const double *src, const int32_t *idx, double *out, long n) {
+  tpx_launch<k_take>(grid1(n), kBlock, 0, c->stream, src, idx, out, n);
+  TPX_LAUNCH_CHECK();
+}
+
 void adjoint_tape_substep(tpx_ctx *c, int rk, const double *const ru_int[3], const double *rho_int) {
   AdjointTape &t = c->adj;
   if (t.step < 0) return;
@@ -810,33 +838,31 @@ void adjoint_reverse(tpx_ctx *c, const GasSweep *gas) {
   }
   // the start of every step of the checkpoint segment being reversed,
   // recomputed once per segment from its checkpoint
-  if (gas && !t.lb) {
-    if (hipMalloc((void **)&t.lb, sizeof(double) * nq * (size_t)np) != hipSuccess ||
-        hipMalloc((void **)&t.lnext, sizeof(double) * nq * (size_t)np) != hipSuccess)
-      throw std::bad_alloc();
-  }
-  if (gas && !t.lug) {  // the pull-form transposes: per-particle adjoints and position bins
-    if (hipMalloc((void **)&t.lug, sizeof(double) * 3 * (size_t)np) != hipSuccess ||
-        hipMalloc((void **)&t.gt, sizeof(double) * (size_t)np) != hipSuccess ||
-        hipMalloc((void **)&t.bkey, sizeof(int32_t) * (size_t)np) != hipSuccess ||
-        hipMalloc((void **)&t.bperm, sizeof(int32_t) * (size_t)np) != hipSuccess ||
-        hipMalloc((void **)&t.binv, sizeof(int32_t) * (size_t)np) != hipSuccess ||
-        hipMalloc((void **)&t.bstart, sizeof(int32_t) * ((size_t)c->g.n + 1)) != hipSuccess)
-      throw std::bad_alloc();
+  auto alloc = [&](auto **p, size_t count) {
+    if (*p) return;
+    *p = static_cast<std::remove_reference_t<decltype(**p)> *>(tape_alloc(t, sizeof(**p) * count));
+    if (!*p) throw std::bad_alloc();
+  };
+  if (gas) {
+    alloc(&t.lb, nq * (size_t)np);
+    alloc(&t.lnext, nq * (size_t)np);
+    // the pull-form transposes: per-particle adjoints and position bins
+    alloc(&t.lug, 3 * (size_t)np);
+    alloc(&t.gt, (size_t)np);
+    alloc(&t.bkey, (size_t)np);
+    alloc(&t.bperm, (size_t)np);
+    alloc(&t.binv, (size_t)np);
+    alloc(&t.bstart, (size_t)c->g.n + 1);
   }
   const int seg_len = std::min(t.every, t.nsteps);
   // the start of every step of the segment and the result of its last; when
   // memory allows, also the four stage states of every step of the segment,
   // kept from the segment's one recomputation (else each step's stages are
   // recomputed from its start when it is reversed)
-  if (!t.seg && hipMalloc((void **)&t.seg, sizeof(double) * nq * (size_t)np * (seg_len + 1)) != hipSuccess)
-    throw std::bad_alloc();
+  alloc(&t.seg, nq * (size_t)np * (seg_len + 1));
   if (!t.segstage && !t.segstage_tried) {
     t.segstage_tried = true;
-    if (hipMalloc((void **)&t.segstage, sizeof(double) * 4 * nq * (size_t)np * seg_len) != hipSuccess) {
-      (void)hipGetLastError();
-      t.segstage = nullptr;
-    }
+    t.segstage = (double *)tape_alloc(t, sizeof(double) * 4 * nq * (size_t)np * seg_len);
   }
   const double *in[7] = {};
   double *out[7] = {};

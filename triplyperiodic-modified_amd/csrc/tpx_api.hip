@@ -681,26 +681,39 @@ void step_end(tpx_ctx *c) {
   do_time_advance(c, true);
 }
 
-// frees every array of a recorded adjoint run
+// The arrays of a recorded adjoint run go back to the tape's blocks
+// (adjoint_free), which the next recording's take.
+// Gives the unused blocks of a tape back to the device (min_idle: those unused
+// over so many recordings)
+void tape_give_back(AdjointTape &t, int min_idle) {
+  size_t m = 0;
+  for (AdjointTape::Block &b : t.blocks) {
+    if (!b.used && b.idle >= min_idle) (void)hipFree(b.p);
+    else t.blocks[m++] = b;
+  }
+  t.blocks.resize(m);
+}
+
 void adjoint_free(AdjointTape &t) {
-  auto f = [](double *&p) { if (p) (void)hipFree(p); p = nullptr; };
+  auto f = [](auto *&p) { p = nullptr; };
   f(t.gas); f(t.ckpt); f(t.y); f(t.seg); f(t.lb); f(t.lnext); f(t.S); f(t.stage); f(t.lam); f(t.dtau); f(t.djdc);
   f(t.start); f(t.final_state); f(t.work); f(t.cap); f(t.lup); f(t.iters_seen); f(t.sub); f(t.tau0);
   f(t.qt); f(t.qs); f(t.p0t); f(t.eps0); f(t.deps); f(t.lh); f(t.hpart); f(t.scal_save); f(t.gck);
+  f(t.cum); f(t.cum_tmp); f(t.lug); f(t.gt); f(t.segstage); f(t.bkey); f(t.bperm); f(t.binv); f(t.bstart);
+  t.pcap.clear();
+  for (AdjointTape::Block &b : t.blocks) {
+    b.idle = b.used ? 0 : b.idle + 1;
+    b.used = false;
+  }
+  tape_give_back(t, 2);
   t.heat = false;
   t.segmented = false;
   t.gas_base = 0;
   t.seg_loaded = -1;
   t.nq = 6;
   t.swept = false;
-  auto fi = [](int32_t *&p) { if (p) (void)hipFree(p); p = nullptr; };
-  fi(t.cum); fi(t.cum_tmp);
-  f(t.lug); f(t.gt); f(t.segstage);
   t.segstage_tried = false;
-  fi(t.bkey); fi(t.bperm); fi(t.binv); fi(t.bstart);
   t.store = false;
-  for (auto &p : t.pcap) f(p);
-  t.pcap.clear();
   t.ga = GasAdjoint{};
   t.ready = false;
 }
@@ -720,6 +733,7 @@ void release(tpx_ctx *c) {
   f(c->scal); f(c->partials); f(c->scan_tmp); f(c->st_part);
   for (auto &p : c->ps) f(p);
   adjoint_free(c->adj);
+  tape_give_back(c->adj, 0);
   if (c->h_scal) (void)hipHostFree(c->h_scal);  // with h_iter and stage.pin[0]
   for (int t = 0; t < kStageMaxThreads; ++t) {
     if (t > 0 && c->stage.pin[t]) (void)hipHostFree(c->stage.pin[t]);
@@ -770,6 +784,29 @@ void timing_begin(tpx_ctx *c, int cls) {
   }
   hip_check(hipEventRecord(a, c->stream), "hipEventRecord");
   t.recs.push_back({cls, a, b});
+}
+
+void *tape_alloc(AdjointTape &t, size_t bytes) {
+  bytes = std::max<size_t>(bytes, 1);
+  AdjointTape::Block *best = nullptr;  // the smallest that fits without wasting much
+  for (AdjointTape::Block &b : t.blocks)
+    if (!b.used && b.bytes >= bytes && b.bytes <= bytes + bytes / 4 + 65536 && (!best || b.bytes < best->bytes)) best = &b;
+  if (best) {
+    best->used = true;
+    best->idle = 0;
+    return best->p;
+  }
+  void *p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    tape_give_back(t, 0);
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+  }
+  t.blocks.push_back({p, bytes, true, 0});
+  return p;
 }
 
 void timing_end(tpx_ctx *c, int cls) {
@@ -1678,15 +1715,15 @@ void gas_state_copy(tpx_ctx *c, double *dst, bool save) {
   if (!save && c->rho_int != c->rho_base) launch_copy(c, c->rho[c->rho_int], dst + 6 * n, n);
 }
 
-// One pool buffer of n values (grown on demand); null when out of memory.
+// Buffer i of n values for the P iterates (grown on demand, 16 at a time where
+// the memory is there); null when out of memory.
 double *pcap_slot(AdjointTape &t, size_t i, long n) {
   while (t.pcap.size() <= i) {
-    double *p = nullptr;
-    if (hipMalloc((void **)&p, sizeof(double) * n) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
-    t.pcap.push_back(p);
+    size_t m = 16;
+    double *p = (double *)tape_alloc(t, sizeof(double) * m * n);
+    if (!p) p = (double *)tape_alloc(t, sizeof(double) * (m = 1) * n);
+    if (!p) return nullptr;
+    for (size_t k = 0; k < m; ++k) t.pcap.push_back(p + k * n);
   }
   return t.pcap[i];
 }
@@ -1752,8 +1789,7 @@ void gas_substeps(tpx_ctx *c, int s, GasSubstep sub[4], bool segment) {
     g.rho_new = cp + 3 * n;
     const double *rn[3];
     ru_ptrs(c, c->ru_new, rn);
-    launch_div_rhs(c, k, 0, rn, c->rho[c->rho_new], t.heat ? g.Q : (c->q_zero ? nullptr : c->Q), nullptr, c->rhs);
-    launch_copy(c, cp + 4 * n, c->rhs, n);
+    launch_div_rhs(c, k, 0, rn, c->rho[c->rho_new], t.heat ? g.Q : (c->q_zero ? nullptr : c->Q), nullptr, cp + 4 * n);
     g.rhs = cp + 4 * n;
     double *sum = segment ? t.sub + (long)t.tape_steps() * 20 * n + (long)j * 4 + rk : t.cap + 20 * n + rk;
     launch_copy(c, sum, c->scal + SC_SUM_RHS, 1);
@@ -1776,7 +1812,7 @@ void gas_substeps(tpx_ctx *c, int s, GasSubstep sub[4], bool segment) {
       double *out = c->P;
       if (it + 1 < g.iters && !(out = pcap_slot(t, used, n))) throw std::bad_alloc();
       c->iter_ctl.first = it == 0;
-      launch_poisson_iteration_on(c, c->rho[c->rho_new], buf, c->rhs, c->scal, nullptr, SC_SUM_RHS, out);
+      launch_poisson_iteration_on(c, c->rho[c->rho_new], buf, g.rhs, c->scal, nullptr, SC_SUM_RHS, out);
       c->iter_ctl.first = 0;
     }
     launch_copy(c, t.iters_seen + (long)s * 4 + rk, c->scal + SC_ITERS, 1);
@@ -1868,8 +1904,8 @@ void taped_step(tpx_ctx *c, int s, GasSubstep sub[4]) {
 void gas_adjoint_run(tpx_ctx *c) {
   AdjointTape &t = c->adj;
   const long n = c->g.n;
-  auto alloc = [](double **p, size_t count) {
-    if (!*p && hipMalloc((void **)p, sizeof(double) * count) != hipSuccess) throw std::bad_alloc();
+  auto alloc = [&](double **p, size_t count) {
+    if (!*p && !(*p = (double *)tape_alloc(t, sizeof(double) * count))) throw std::bad_alloc();
   };
   alloc(&t.work, (size_t)GasAdjoint::kFields * n + SC_COUNT);
   alloc(&t.lup, 3 * (size_t)n);
@@ -1939,20 +1975,6 @@ void gas_adjoint_run(tpx_ctx *c) {
   sync(c);
   for (size_t q = 0; q < seen.size(); ++q)
     if ((int)seen[q] != t.iters[q]) throw std::logic_error("adjoint: a recomputed Poisson solve differs from the recorded one");
-}
-
-// host copy of the sum of device arrays (n values each)
-void download_sum(tpx_ctx *c, std::initializer_list<const double *> src, double *dst) {
-  const size_t n = (size_t)c->g.n;
-  std::vector<double> tmp(n);
-  bool first = true;
-  for (const double *p : src) {
-    const HostPart part{first ? dst : tmp.data(), p, sizeof(double) * n};
-    download(c, &part, 1);
-    if (!first)
-      for (size_t q = 0; q < n; ++q) dst[q] += tmp[q];
-    first = false;
-  }
 }
 
 }  // namespace
@@ -2080,8 +2102,9 @@ int tpx_adjoint_record(tpx_ctx *ctx, int nsteps, int every, double *J) {
     t.nq = t.heat ? 7 : 6;
     const long n = c->g.n, np = pt.n;
     const size_t nq = (size_t)t.nq;
-    auto alloc = [](double **p, size_t count) {
-      if (hipMalloc((void **)p, sizeof(double) * count) != hipSuccess) throw std::bad_alloc();
+    auto alloc = [&](auto **p, size_t count) {
+      *p = static_cast<std::remove_reference_t<decltype(**p)> *>(tape_alloc(t, sizeof(**p) * count));
+      if (!*p) throw std::bad_alloc();
     };
     t.segmented = t.mode == 3;
     t.gas_base = 0;
@@ -2108,9 +2131,8 @@ int tpx_adjoint_record(tpx_ctx *ctx, int nsteps, int every, double *J) {
     }
     alloc(&t.dtau, (size_t)np);
     alloc(&t.djdc, (size_t)n);
-    if (hipMalloc((void **)&t.cum, sizeof(int32_t) * np) != hipSuccess ||
-        hipMalloc((void **)&t.cum_tmp, sizeof(int32_t) * np) != hipSuccess)
-      throw std::bad_alloc();
+    alloc(&t.cum, (size_t)np);
+    alloc(&t.cum_tmp, (size_t)np);
     launch_iota(c, t.cum, np);
     if (pt.has_tau) {
       alloc(&t.tau0, (size_t)np);
@@ -2128,15 +2150,13 @@ int tpx_adjoint_record(tpx_ctx *ctx, int nsteps, int every, double *J) {
     if (t.mode == 0 || t.mode == 1) {
       size_t free_b = 0, total_b = 0;
       hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+      for (const AdjointTape::Block &b : t.blocks)
+        if (!b.used) free_b += b.bytes;
       const double need = (double)nsteps * 4 * (5 + 3) * n * sizeof(double);
       if (t.mode == 1 || need < 0.5 * (double)free_b) {
-        t.store = hipMalloc((void **)&t.sub, sizeof(double) * ((size_t)nsteps * 20 * n + (size_t)nsteps * 4)) ==
-                  hipSuccess;
-        if (!t.store) {
-          (void)hipGetLastError();
-          t.sub = nullptr;
-          if (t.mode == 1) throw std::bad_alloc();
-        }
+        t.sub = (double *)tape_alloc(t, sizeof(double) * ((size_t)nsteps * 20 * n + (size_t)nsteps * 4));
+        t.store = t.sub != nullptr;
+        if (!t.store && t.mode == 1) throw std::bad_alloc();
       }
     }
     t.g3.assign((size_t)nsteps * 3, 0.0);
@@ -2145,6 +2165,19 @@ int tpx_adjoint_record(tpx_ctx *ctx, int nsteps, int every, double *J) {
     t.iteration.assign((size_t)nsteps, 0);
     t.iters.assign((size_t)nsteps * 4, 0);
     adjoint_checkpoint(c, 0);
+    // what the sweep reads of the drag and heat deposits and the Poisson
+    // right-hand side is written by their kernels straight into the tape: the
+    // context's arrays stand aside while the run is recorded
+    struct Aside {
+      tpx_ctx *c;
+      double *S[3], *Q, *rhs;
+      explicit Aside(tpx_ctx *ctx) : c(ctx), S{ctx->S[0], ctx->S[1], ctx->S[2]}, Q(ctx->Q), rhs(ctx->rhs) {}
+      ~Aside() {
+        for (int d = 0; d < 3; ++d) c->S[d] = S[d];
+        c->Q = Q;
+        c->rhs = rhs;
+      }
+    } aside(c);
     try {
       for (int s = 0; s < nsteps; ++s) {
         t.step = s;
@@ -2171,19 +2204,17 @@ int tpx_adjoint_record(tpx_ctx *ctx, int nsteps, int every, double *J) {
         t.iteration[s] = c->Iteration;
         for (int d = 0; d < 3; ++d) t.gv[(size_t)s * 3 + d] = c->gv[d];
         for (int rk = 0; rk < 4; ++rk) {  // fused_substep, keeping each solve's iteration count
-          fused_substep_pre(c, rk);
           const size_t q = (size_t)s * 4 + rk;
           if (twc)
-            for (int d = 0; d < 3; ++d) launch_copy(c, t.S + ((long)q * 3 + d) * n, c->S[d], n);
-          if (t.heat) {
-            launch_copy(c, t.qt + (long)q * n, c->Q, n);
-            launch_copy(c, t.qs + q, c->scal + SC_SUM_Q, 1);
-          }
+            for (int d = 0; d < 3; ++d) c->S[d] = t.S + ((long)q * 3 + d) * n;
+          if (t.heat) c->Q = t.qt + (long)q * n;
+          c->rhs = t.store ? t.sub + ((long)q * 5 + 4) * n : aside.rhs;
+          fused_substep_pre(c, rk);
+          if (t.heat) launch_copy(c, t.qs + q, c->scal + SC_SUM_Q, 1);
           if (t.store) {  // what the gas sweep reads, so that it need not recompute the step
             double *dst = t.sub + (long)q * 5 * n;
             for (int d = 0; d < 3; ++d) launch_copy(c, dst + d * n, c->ru[c->ru_new][d], n);
             launch_copy(c, dst + 3 * n, c->rho[c->rho_new], n);
-            launch_copy(c, dst + 4 * n, c->rhs, n);
             launch_copy(c, t.sub + (long)nsteps * 20 * n + q, c->scal + SC_SUM_RHS, 1);
           }
           const size_t p0 = t.pnext;
@@ -2209,6 +2240,10 @@ int tpx_adjoint_record(tpx_ctx *ctx, int nsteps, int every, double *J) {
       t.step = -1;
       throw;
     }
+    if (twc)
+      for (int d = 0; d < 3; ++d) launch_copy(c, aside.S[d], c->S[d], n);
+    if (t.heat) launch_copy(c, aside.Q, c->Q, n);
+    if (c->rhs != aside.rhs) launch_copy(c, aside.rhs, c->rhs, n);
     gas_state_copy(c, t.final_state, true);
     if (t.heat) launch_copy(c, t.p0t + (long)nsteps * 4, c->scal + SC_P0, 1);
     const double j = adjoint_objective(c);
@@ -2235,33 +2270,34 @@ int tpx_adjoint_gradient_full(tpx_ctx *ctx, double *dJ_dtau, double *dJ_dstate, 
     if (gas || ctx->p.twc || t.heat || t.segmented) gas_adjoint_run(ctx);
     else adjoint_reverse(ctx, nullptr);
     const size_t np = (size_t)ctx->pt.n, n = (size_t)ctx->g.n;
-    // the sweep's particle arrays are in the recording's order: give them in
-    // the context's present order (cum maps the one to the other)
-    std::vector<int32_t> cum(np);
-    std::vector<double> tmp(6 * np);
-    hip_check(hipMemcpyAsync(cum.data(), t.cum, sizeof(int32_t) * np, hipMemcpyDeviceToHost, ctx->stream), "download");
-    if (dJ_dtau)
-      hip_check(hipMemcpyAsync(tmp.data(), t.dtau, sizeof(double) * np, hipMemcpyDeviceToHost, ctx->stream), "download");
-    sync(ctx);
-    if (dJ_dtau)
-      for (size_t i = 0; i < np; ++i) dJ_dtau[i] = tmp[(size_t)cum[i]];
-    if (dJ_dstate) {  // adjoint of the recorded run's initial x, y, z, u, v, w (the first 6 rows)
-      hip_check(hipMemcpyAsync(tmp.data(), t.lam, sizeof(double) * 6 * np, hipMemcpyDeviceToHost, ctx->stream),
-                "download");
-      sync(ctx);
-      for (int q = 0; q < 6; ++q)
-        for (size_t i = 0; i < np; ++i) dJ_dstate[q * np + i] = tmp[q * np + (size_t)cum[i]];
-    }
-    if (dJ_dA)
-      hip_check(hipMemcpyAsync(dJ_dA, ctx->scal + SC_ADJ_A, sizeof(double), hipMemcpyDeviceToHost, ctx->stream),
-                "download");
-    sync(ctx);
+    // the sweep's particle arrays are in the recording's order: given in the
+    // context's present order (cum maps the one to the other), gathered into
+    // the spent stage states; the recorded run starts with RU_int = RU_np1 = RU
+    // and Rho_int = Rho_np1 = Rho, whose adjoints add up (into spent work)
+    HostPart part[13];
+    int m = 0;
+    double *take = t.stage;
+    auto give = [&](const double *src, double *dst) {
+      launch_take(ctx, src, t.cum, take, (long)np);
+      part[m++] = {dst, take, sizeof(double) * np};
+      take += np;
+    };
+    if (dJ_dtau) give(t.dtau, dJ_dtau);
+    if (dJ_dstate)  // adjoint of the recorded run's initial x, y, z, u, v, w (the first 6 rows)
+      for (int q = 0; q < 6; ++q) give(t.lam + q * np, dJ_dstate + q * np);
+    if (dJ_dA) part[m++] = {dJ_dA, ctx->scal + SC_ADJ_A, sizeof(double)};
     const GasAdjoint &ga = t.ga;
-    // the recorded run starts with RU_int = RU_np1 = RU and Rho_int = Rho_np1 = Rho
     if (dJ_dRU)
-      for (int d = 0; d < 3; ++d) download_sum(ctx, {ga.lru[d], ga.lnp1[d], ga.lint[d]}, dJ_dRU + d * n);
-    if (dJ_dRho) download_sum(ctx, {ga.lr, ga.lrnp1, ga.lrint}, dJ_dRho);
-    if (dJ_dP) download_sum(ctx, {ga.lp}, dJ_dP);
+      for (int d = 0; d < 3; ++d) {
+        launch_sum3(ctx, ga.lru[d], ga.lnp1[d], ga.lint[d], ga.lF[d], (long)n);
+        part[m++] = {dJ_dRU + d * n, ga.lF[d], sizeof(double) * n};
+      }
+    if (dJ_dRho) {
+      launch_sum3(ctx, ga.lr, ga.lrnp1, ga.lrint, ga.lrhs_p, (long)n);
+      part[m++] = {dJ_dRho, ga.lrhs_p, sizeof(double) * n};
+    }
+    if (dJ_dP) part[m++] = {dJ_dP, ga.lp, sizeof(double) * n};
+    download(ctx, part, m);
     return TPX_OK;
   });
 }
@@ -2274,17 +2310,16 @@ int tpx_adjoint_gradient_heat(tpx_ctx *ctx, double *dJ_dT, double *dJ_deps, doub
     if (!dJ_dT && !dJ_deps && !dJ_dP0) throw std::invalid_argument("null outputs");
     if (!t.swept) gas_adjoint_run(ctx);
     const size_t np = (size_t)ctx->pt.n;
-    std::vector<int32_t> cum(np);
-    std::vector<double> tmp(np);
-    hip_check(hipMemcpyAsync(cum.data(), t.cum, sizeof(int32_t) * np, hipMemcpyDeviceToHost, ctx->stream), "download");
-    sync(ctx);
+    HostPart part[2];
+    int m = 0;
     auto give = [&](const double *src, double *dst) {  // in the context's present particle order
-      hip_check(hipMemcpyAsync(tmp.data(), src, sizeof(double) * np, hipMemcpyDeviceToHost, ctx->stream), "download");
-      sync(ctx);
-      for (size_t i = 0; i < np; ++i) dst[i] = tmp[(size_t)cum[i]];
+      double *take = t.stage + m * np;
+      launch_take(ctx, src, t.cum, take, (long)np);
+      part[m++] = {dst, take, sizeof(double) * np};
     };
     if (dJ_dT) give(t.lam + 6 * np, dJ_dT);
     if (dJ_deps) give(t.deps, dJ_deps);
+    download(ctx, part, m);
     if (dJ_dP0) {  // the initial P0 is both P0 and P0_np1 of the first step, and fed its first exchange
       double sc[SC_ADJ_P0I - SC_ADJ_P0 + 1];
       hip_check(hipMemcpyAsync(sc, ctx->scal + SC_ADJ_P0, sizeof(sc), hipMemcpyDeviceToHost, ctx->stream), "download");
@@ -2308,6 +2343,7 @@ int tpx_adjoint_release(tpx_ctx *ctx) {
   return guarded(ctx, [&]() {
     sync(ctx);
     adjoint_free(ctx->adj);
+    tape_give_back(ctx->adj, 0);
     return TPX_OK;
   });
 }

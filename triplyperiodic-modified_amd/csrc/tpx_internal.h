@@ -207,6 +207,11 @@ struct AdjointTape {
   std::vector<double> I0;        // lamp intensity of each step
   bool swept = false;            // a sweep has run since the recording
   GasAdjoint ga{};
+  // device memory of the arrays above, kept from one recording to the next (a
+  // recording's allocations and frees took longer than its steps) and given
+  // back on release, when the device is full, or unused over two recordings
+  struct Block { void *p; size_t bytes; bool used; int idle; };
+  std::vector<Block> blocks;
   // steps the gas and sub tapes hold
   int tape_steps() const { return segmented ? std::min(every, nsteps) : nsteps; }
   // the gas tape of step s (4 substeps x 4 fields of n)
@@ -426,7 +431,13 @@ void launch_bin_by_key(tpx_ctx *c, const int32_t *key, int32_t *perm, int32_t *i
 void launch_zero_counts(tpx_ctx *c, int32_t *cnt);
 void launch_exclusive_scan(tpx_ctx *c, int32_t *data, int64_t n);  // in place
 
+// memory of the adjoint's arrays (tpx_api.hip): null when the device is full
+void *tape_alloc(AdjointTape &t, size_t bytes);
+
 // k_adjoint.hip
+// out = (a + b) + c and out[i] = src[idx[i]] (the sweep's outputs)
+void launch_sum3(tpx_ctx *c, const double *a, const double *b, const double *d, double *out, long n);
+void launch_take(tpx_ctx *c, const double *src, const int32_t *idx, double *out, long n);
 void adjoint_tape_substep(tpx_ctx *c, int rk, const double *const ru_int[3], const double *rho_int);
 void adjoint_checkpoint(tpx_ctx *c, int slot);
 void adjoint_track_permutation(tpx_ctx *c);  // before a re-sort by pt.perm_int during a recording

@@ -316,8 +316,8 @@ class Solver:
         the gas where the recorded run ended."""
         n = ctypes.c_int64()
         self._ok(self.L.tpx_num_particles(self.h, ctypes.byref(n)), "num_particles")
-        out = dict(tau=np.zeros(n.value), state=np.zeros((6, n.value)), A=np.zeros(1),
-                   RU=np.zeros((3,) + self.shape), Rho=np.zeros(self.shape), P=np.zeros(self.shape))
+        out = dict(tau=np.empty(n.value), state=np.empty((6, n.value)), A=np.zeros(1),
+                   RU=np.empty((3,) + self.shape), Rho=np.empty(self.shape), P=np.empty(self.shape))
         self._ok(self.L.tpx_adjoint_gradient_full(self.h, _dp(out["tau"]), _dp(out["state"]), _dp(out["A"]),
                                                   _dp(out["RU"]), _dp(out["Rho"]), _dp(out["P"])),
                  "adjoint_gradient_full")
@@ -340,7 +340,7 @@ class Solver:
         since the recording)."""
         n = ctypes.c_int64()
         self._ok(self.L.tpx_num_particles(self.h, ctypes.byref(n)), "num_particles")
-        out = dict(T=np.zeros(n.value), eps=np.zeros(n.value), P0=np.zeros(1))
+        out = dict(T=np.empty(n.value), eps=np.empty(n.value), P0=np.zeros(1))
         self._ok(self.L.tpx_adjoint_gradient_heat(self.h, _dp(out["T"]), _dp(out["eps"]), _dp(out["P0"])),
                  "adjoint_gradient_heat")
         out["P0"] = float(out["P0"][0])
