@@ -28,7 +28,8 @@ def _case(shape):
 
 
 @pytest.mark.parametrize("shape", [(16, 16, 16), (32, 16, 32), (16, 64, 64), (64, 16, 128), (16, 32, 256), (256, 32, 16),
-                                   (16, 8, 64), (512, 16, 16)])
+                                   (16, 8, 64), (512, 16, 16), (16, 16, 512), (16, 512, 32), (512, 128, 16),
+                                   (16, 512, 512), (32, 256, 512)])
 def test_three_pass_coefficient_solve_equals_five_pass(gpu_available, monkeypatch, shape):
     p, C, RHS, P0 = _case(shape)
     out = []

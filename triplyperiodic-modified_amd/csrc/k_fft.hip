@@ -5,9 +5,10 @@
 //   r  = (div_F2C(C grad_C2F P) - RHS) * cc,   C = 1/Rho_face, cc = -1/I_F2C(C)
 //   dp = -Re IFFT( FFT(r) / lambda(k) ) / N^3   (zero mode passed through)
 //   P += dp,  err = max|dp|
-// with r real.  When every axis length is 16..256 the iteration is three
-// passes over the half spectrum (k_xy_fwd, k_yz_pass, k_xy_inv below: the y
-// transform is split between them along its four-step factorisation).
+// with r real.  When every axis length is 16..512 (y and z not both 512) the
+// iteration is three passes over the half spectrum (k_xy_fwd, k_yz_pass,
+// k_xy_inv below: the y transform is split between them along its four-step
+// factorisation).
 // Otherwise it is five:
 //   X  (forward): residual computed in registers, real-to-half-complex FFT
 //                 along x; only kx = 0..nx/2 is stored ((nx/2+1) ny nz).
@@ -16,12 +17,13 @@
 //   Y  (inverse).
 //   X  (inverse): Hermitian extension, inverse FFT along x, P += dp and the
 //                 block maxima of |dp|.
-// Axis lengths 16..256 use four-step register kernels (n = R1 R2, one LDS
+// There, lengths 16..256 use four-step register kernels (n = R1 R2, one LDS
 // exchange); 8 and 512 use LDS Stockham kernels.  C and cc are recomputed
 // from Rho_new in the X pass instead of being stored.
 #include <math.h>
 
 #include <algorithm>
+#include <initializer_list>
 #include <stdexcept>
 #include <vector>
 
@@ -459,8 +461,8 @@ struct k_zpass {
 };
 
 // ---------------------------------------------------------------------------
-// Four-step register FFT for lines of n = R1 * R2 points (R1 >= R2, both in
-// {4, 8, 16}).  With i = t + R1 m and k = k2 + R2 k1,
+// Four-step register FFT for lines of n = R1 * R2 points (R1 >= R2, in
+// {4, 8, 16, 32}).  With i = t + R1 m and k = k2 + R2 k1,
 //   X[k2 + R2 k1] = sum_t W_R1^{t k1} W_n^{t k2} sum_m x[t + R1 m] W_R2^{m k2}.
 // Step A: the work item for t holds x[t + R1 m] (m < R2) in registers,
 //         transforms over m and applies W_n^{t k2}.
@@ -598,6 +600,37 @@ struct RegDft<16, INV> {
     for (int k1 = 0; k1 < 4; ++k1)
 #pragma unroll
       for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = y[4 * k1 + k2];
+  }
+};
+
+// e^{-2 pi i k/32}, k < 16
+__device__ __forceinline__ double2 w32(int k) {
+  constexpr double c[9] = {1.0, 0.9807852804032304, 0.9238795325112867, 0.8314696123025452, 0.7071067811865476,
+                           0.5555702330196022, 0.3826834323650898, 0.1950903220161283, 0.0};  // cos(pi q/16)
+  return k <= 8 ? make_double2(c[k], -c[8 - k]) : make_double2(-c[16 - k], -c[k - 8]);
+}
+
+// 32 = 2 x 16: 16-point transforms of the even and the odd points, the
+// twiddles W_32^{k1}, radix-2
+template <bool INV>
+struct RegDft<32, INV> {
+  static __device__ __forceinline__ void run(double2 *v) {
+    double2 e[16], o[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      e[q] = v[2 * q];
+      o[q] = v[2 * q + 1];
+    }
+    RegDft<16, INV>::run(e);
+    RegDft<16, INV>::run(o);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      double2 w = w32(q);
+      if (INV) w.y = -w.y;
+      const double2 t = q == 0 ? o[q] : cmul(o[q], w);
+      v[q] = cadd(e[q], t);
+      v[q + 16] = csub(e[q], t);
+    }
   }
 };
 
@@ -860,7 +893,7 @@ struct k_zpass4 {
 };
 
 // ---------------------------------------------------------------------------
-// Three-pass iteration (every axis length 16..256).  The y transform is split
+// Three-pass iteration (axis lengths 16..512).  The y transform is split
 // between the passes along its four-step factorisation ny = Y1 Y2, with
 // y = t + Y1 m:
 //   pass 1, block (z, t):   residual and x transform of the Y2 rows
@@ -966,7 +999,7 @@ struct k_yz_pass {
   // and Y1 = 8 (the 64^3 boxes), where 256 would leave three waves of four idle
   // in every transform stage
   static constexpr int kItems = std::max(Z1 * Z2, Y1 * std::max(Z1, Z2));
-  static constexpr int kBounds = kItems <= 64 ? 64 : (kItems <= 128 ? 128 : 256);
+  static constexpr int kBounds = kItems <= 64 ? 64 : (kItems <= 128 ? 128 : (kItems <= 256 ? 256 : 512));
   static __device__ __forceinline__ void run(double2 *spec, int mxh, int Y2, const double2 *__restrict__ twz,
                                                  const double *__restrict__ lamx,
                                                  const double *__restrict__ lamy,
@@ -1129,7 +1162,7 @@ struct k_yz_pass {
 
 // ---------------------------------------------------------------------------
 // Pass 1 with the x transform of the real residual done as a complex
-// transform of half the length (x lengths 2 M = 64, 128, 256; 16 lanes a row):
+// transform of half the length (x lengths 2 M = 64, 128, 256, 512; 16 lanes a row):
 // lane ta of a row holds the pairs z[j] = x[2j] + i x[2j+1], j = ta + 16 m
 // (m < R2H, M = 16 R2H), loaded with 16-byte accesses.  The M-point four-step
 // transform Z of z gives the half spectrum of x by
@@ -1314,6 +1347,107 @@ struct k_xy_fwd_rp {
 #pragma unroll
       for (int k2 = 0; k2 < Y2; ++k2) dst[k2 * ks] = w[k2];
     }
+  }
+};
+
+// Pass 3 for x length 2 M = 512, the mirror of the packed pass 1: the real row
+// of 2 M points from one complex inverse transform of M,
+//   Z[k] = (X[k] + conj X[M-k]) + i (X[k] - conj X[M-k]) conj(W_2M^k),
+//   z = IFFT_M(Z) = x[2j] + i x[2j+1],
+// P read and written in pairs.  Only 512 takes it: there the 16 x 16 transform
+// keeps every work item busy to the end and the full-length row would need 32
+// points a thread; at 128 and 256 its last stage has items for half the block
+// and it measured slower than the full-length inverse.
+template <int R2H, int Y2, bool Overwrite, bool OutOfPlace>
+struct k_xy_inv_rp {
+  static constexpr int kBounds = 256;
+  static __device__ __forceinline__ void run(const XInvArgs &a, int Y1, const double2 *__restrict__ twy) {
+    if (a.done && *a.done != 0.0) return;  // the solve has converged
+    extern __shared__ double ldsd[];
+    __shared__ double red[256];
+    constexpr int R1 = 16, M = R1 * R2H, P = R1 + 1, SP = Y2 + 1;
+    const Geo &g = a.g;
+    const int mxh = M + 1;
+    const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+    const int t = (int)(blk % (unsigned)Y1), z = (int)(blk / (unsigned)Y1);
+    double2 *S = reinterpret_cast<double2 *>(ldsd);  // S[kx SP + row]
+    const long cs = (long)g.nz * Y1 + kRunPad;
+    const long ks = cs * mxh;
+    for (int kx = threadIdx.x; kx < mxh; kx += block_dim_x()) {
+      const double2 *src = a.spec + kx * cs + z * Y1 + t;
+      double2 w[Y2];
+#pragma unroll
+      for (int k2 = 0; k2 < Y2; ++k2) {
+        w[k2] = src[k2 * ks];
+        if (k2 > 0) {
+          double2 tw = twy[t * k2];
+          tw.y = -tw.y;
+          w[k2] = cmul(w[k2], tw);
+        }
+      }
+      RegDft<Y2, true>::run(w);
+#pragma unroll
+      for (int m = 0; m < Y2; ++m) S[kx * SP + m] = w[m];
+    }
+    __syncthreads();
+    const int tx = threadIdx.x % R1, c = threadIdx.x / R1;
+    double2 v[R2H];
+#pragma unroll
+    for (int m = 0; m < R2H; ++m) {
+      const int k = tx + R1 * m;
+      double2 A = S[k * SP + c], B = S[(M - k) * SP + c];
+      if (k == 0) A.y = B.y = 0.0;  // the real modes 0 and M
+      const double2 w = a.tw[k];
+      const double2 E = make_double2(A.x + B.x, A.y - B.y), D = make_double2(A.x - B.x, A.y + B.y);
+      const double2 O = cmul(D, make_double2(w.x, -w.y));
+      v[m] = make_double2(E.x - O.y, E.y + O.x);
+    }
+    RegDft<R2H, true>::run(v);
+#pragma unroll
+    for (int k2 = 1; k2 < R2H; ++k2) {
+      double2 w = a.tw[2 * tx * k2];
+      w.y = -w.y;
+      v[k2] = cmul(v[k2], w);
+    }
+    __syncthreads();  // S is reused by the exchange
+    const bool b_item = (int)threadIdx.x < Y2 * R2H;
+    const int k2x = threadIdx.x % R2H, cb = threadIdx.x / R2H;
+    double2 u[R1];
+#pragma unroll
+    for (int q = 0; q < R2H; ++q) ldsd[(c * R2H + q) * P + tx] = v[q].x;
+    __syncthreads();
+    if (b_item) {
+#pragma unroll
+      for (int q = 0; q < R1; ++q) u[q].x = ldsd[(cb * R2H + k2x) * P + q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < R2H; ++q) ldsd[(c * R2H + q) * P + tx] = v[q].y;
+    __syncthreads();
+    double mx = 0.0;
+    if (b_item) {
+#pragma unroll
+      for (int q = 0; q < R1; ++q) u[q].y = ldsd[(cb * R2H + k2x) * P + q];
+      RegDft<R1, true>::run(u);
+      const long l0 = ((long)z * g.ny + t + Y1 * cb) * (2 * M) + 2 * k2x;
+      const double *Pi = a.P + l0;
+      double *Po = (OutOfPlace ? a.Pout : a.P) + l0;
+#pragma unroll
+      for (int k1 = 0; k1 < R1; ++k1) {
+        const double2 dp = make_double2((-1) * u[k1].x / (a.ncell), (-1) * u[k1].y / (a.ncell));
+        double2 q = dp;
+        if constexpr (!Overwrite) q = cadd(*reinterpret_cast<const double2 *>(Pi + 2 * R2H * k1), dp);
+        *reinterpret_cast<double2 *>(Po + 2 * R2H * k1) = q;
+        mx = fmax(mx, fmax(fabs(dp.x), fabs(dp.y)));
+      }
+    }
+    red[threadIdx.x] = mx;
+    __syncthreads();
+    for (int s = block_dim_x() / 2; s > 0; s >>= 1) {
+      if ((int)threadIdx.x < s) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + s]);
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) a.partials[blk] = red[0];
   }
 };
 
@@ -1570,7 +1704,7 @@ void xy_fwd_launch(unsigned nb, size_t sh, hipStream_t st, const XArgs &xa, int 
   if (xa.cf[0]) xy_fwd_launch_t<R1, R2, true>(nb, sh, st, xa, Y1, Y2, twy);
   else xy_fwd_launch_t<R1, R2, false>(nb, sh, st, xa, Y1, Y2, twy);
 }
-// the packed forward form for x lengths 64, 128 and 256 (R2H = 2, 4, 8)
+// the packed forward form for x lengths 64, 128, 256 and 512 (R2H = 2, 4, 8, 16)
 template <int R2H, bool Coef>
 void xy_fwd_rp_launch_t(unsigned nb, size_t sh, hipStream_t st, const XArgs &xa, int Y1, int Y2, const double2 *twy) {
   switch (Y2) {
@@ -1592,6 +1726,19 @@ void xy_inv_launch_t(unsigned nb, size_t sh, hipStream_t st, const XInvArgs &xi,
     default: tpx_launch<k_xy_inv<R1, R2, 16, Ow, Oop>>(nb, 16 * R1, sh, st, xi, Y1, twy); break;
   }
 }
+template <bool Ow, bool Oop>
+void xy_inv_rp_launch_t(unsigned nb, size_t sh, hipStream_t st, const XInvArgs &xi, int Y1, int Y2, const double2 *twy) {
+  switch (Y2) {
+    case 4: tpx_launch<k_xy_inv_rp<16, 4, Ow, Oop>>(nb, 4 * 16, sh, st, xi, Y1, twy); break;
+    case 8: tpx_launch<k_xy_inv_rp<16, 8, Ow, Oop>>(nb, 8 * 16, sh, st, xi, Y1, twy); break;
+    default: tpx_launch<k_xy_inv_rp<16, 16, Ow, Oop>>(nb, 16 * 16, sh, st, xi, Y1, twy); break;
+  }
+}
+void xy_inv_rp_launch(unsigned nb, size_t sh, hipStream_t st, const XInvArgs &xi, int Y1, int Y2, const double2 *twy) {
+  if (xi.overwrite) xy_inv_rp_launch_t<true, false>(nb, sh, st, xi, Y1, Y2, twy);
+  else if (xi.Pout) xy_inv_rp_launch_t<false, true>(nb, sh, st, xi, Y1, Y2, twy);
+  else xy_inv_rp_launch_t<false, false>(nb, sh, st, xi, Y1, Y2, twy);
+}
 template <int R1, int R2>
 void xy_inv_launch(unsigned nb, size_t sh, hipStream_t st, const XInvArgs &xi, int Y1, int Y2, const double2 *twy) {
   if (xi.overwrite) xy_inv_launch_t<R1, R2, true, false>(nb, sh, st, xi, Y1, Y2, twy);
@@ -1607,11 +1754,18 @@ size_t yz_shared_bytes(int y1, int nz) {
 template <int Z1, int Z2>
 void yz_launch(unsigned nb, size_t sh, hipStream_t st, double2 *spec, int mxh, int Y1, int Y2, const tpx_ctx *c,
                const double *done) {
+#define L_YZ1(Y)                                                                                                  \
+  tpx_launch<k_yz_pass<Y, Z1, Z2>>(nb, k_yz_pass<Y, Z1, Z2>::kBounds, sh, st, spec, mxh, Y2, c->tw[2], c->lam[0], \
+                                   c->lam[1], c->lam[2], done)
   switch (Y1) {
-    case 4: tpx_launch<k_yz_pass<4, Z1, Z2>>(nb, k_yz_pass<4, Z1, Z2>::kBounds, sh, st, spec, mxh, Y2, c->tw[2], c->lam[0], c->lam[1], c->lam[2], done); break;
-    case 8: tpx_launch<k_yz_pass<8, Z1, Z2>>(nb, k_yz_pass<8, Z1, Z2>::kBounds, sh, st, spec, mxh, Y2, c->tw[2], c->lam[0], c->lam[1], c->lam[2], done); break;
-    default: tpx_launch<k_yz_pass<16, Z1, Z2>>(nb, k_yz_pass<16, Z1, Z2>::kBounds, sh, st, spec, mxh, Y2, c->tw[2], c->lam[0], c->lam[1], c->lam[2], done); break;
+    case 4: L_YZ1(4); break;
+    case 8: L_YZ1(8); break;
+    case 16: L_YZ1(16); break;
+    default:
+      if constexpr (Z1 * Z2 <= 256) L_YZ1(32);
+      else throw std::logic_error("the run of y and z lengths 512 does not fit in LDS");
   }
+#undef L_YZ1
 }
 
 void launch_solve_state(tpx_ctx *c, double *dst) {
@@ -1635,11 +1789,38 @@ void launch_residual_coef(tpx_ctx *c, const double *const cf[3], const double *P
   TPX_LAUNCH_CHECK();
 }
 
-// Whether one transform pair fits the three-pass form (every axis 16..256);
-// r1, r2 / y1, y2 / z1, z2: the four-step factors of x, y and z.
-bool three_pass_shape(const tpx_ctx *c, int &r1, int &r2, int &y1, int &y2, int &z1, int &z2) {
+bool aligned16(std::initializer_list<const void *> p) {
+  for (const void *q : p)
+    if ((uintptr_t)q % 16 != 0) return false;
+  return true;
+}
+
+// Whether one transform pair fits the three-pass form (lengths of 16..512, y
+// and z not both 512: the run of a pass-2 block would be 278 KB); r1, r2 / y1,
+// y2 / z1, z2: the four-step factors of x, y and z.  An x length of 512 has only
+// the packed rows (16 x 16 points of pairs), which need 16-byte aligned fields:
+// `aligned`.
+// An axis of 512 took the five-pass form with Stockham transforms before; one
+// iteration: 512 x 64 x 128 154 -> 95 us, 64 x 512 x 128 179 -> 124, 64 x 128 x
+// 512 167 -> 116, 128 x 256 x 512 650 -> 469, 512 x 32 x 512 347 -> 205.
+bool three_pass_shape(const tpx_ctx *c, int &r1, int &r2, int &y1, int &y2, int &z1, int &z2, bool aligned = true) {
   const Geo &g = c->g;
-  return c->fft_passes == 3 && four_step(g.nx, r1, r2) && four_step(g.ny, y1, y2) && four_step(g.nz, z1, z2);
+  // 512 = 32 x 16 along y (16 rows a block in passes 1 and 3), 16 x 32 along z
+  // (the division by lambda between two transforms of 16 points, not of 32,
+  // which would spill)
+  auto factors = [](int n, int &f1, int &f2, bool y) {
+    if (n != 512) return four_step(n, f1, f2);
+    f1 = y ? 32 : 16;
+    f2 = y ? 16 : 32;
+    return true;
+  };
+  if (c->fft_passes != 3 || (g.ny == 512 && g.nz == 512) || !factors(g.ny, y1, y2, true) || !factors(g.nz, z1, z2, false))
+    return false;
+  if (g.nx == 512 && c->x_packed && aligned) {
+    r1 = r2 = 16;
+    return true;
+  }
+  return four_step(g.nx, r1, r2);
 }
 
 // The three passes of one transform pair (passes 1 and 3 as xa, xi ask);
@@ -1657,11 +1838,11 @@ unsigned three_pass_launch(tpx_ctx *c, const XArgs &xa, const XInvArgs &xi, cons
   // update, measured slower)
   // the packed form reads pairs with 16-byte loads: the library's own fields
   // are aligned, a caller's arrays (coefficient solve) need not be
-  bool packed = (g.nx == 64 || g.nx == 128 || g.nx == 256) && c->x_packed;
-  if (xa.cf[0])
-    for (const double *q : {xa.cf[0], xa.cf[1], xa.cf[2], xa.P, xa.rhs}) packed = packed && (uintptr_t)q % 16 == 0;
+  bool packed = (g.nx == 64 || g.nx == 128 || g.nx == 256 || g.nx == 512) && c->x_packed;
+  if (xa.cf[0]) packed = packed && aligned16({xa.cf[0], xa.cf[1], xa.cf[2], xa.P, xa.rhs});
 #define L_XYF(A, B) xy_fwd_launch<A, B>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1])
-  if (packed && g.nx == 256) xy_fwd_rp_launch<8>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1]);
+  if (g.nx == 512) xy_fwd_rp_launch<16>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1]);
+  else if (packed && g.nx == 256) xy_fwd_rp_launch<8>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1]);
   else if (packed && g.nx == 128) xy_fwd_rp_launch<4>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1]);
   else if (packed) xy_fwd_rp_launch<2>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1]);
   else { TPX_FOUR_STEP_SWITCH(g.nx, L_XYF) }
@@ -1672,13 +1853,15 @@ unsigned three_pass_launch(tpx_ctx *c, const XArgs &xa, const XInvArgs &xi, cons
   const unsigned nb2 = (unsigned)(mxh * y2);
   const size_t sh2 = yz_shared_bytes(y1, g.nz);
 #define L_YZ(A, B) yz_launch<A, B>(nb2, sh2, c->stream, c->spec[0], mxh, y1, y2, c, done)
-  TPX_FOUR_STEP_SWITCH(g.nz, L_YZ)
+  if (g.nz == 512) L_YZ(16, 32);
+  else { TPX_FOUR_STEP_SWITCH(g.nz, L_YZ) }
 #undef L_YZ
   TPX_LAUNCH_CHECK();
   timing_end(c, TPX_K_FFT_YZ);
   timing_begin(c, TPX_K_FFT_INV);
 #define L_XYI(A, B) xy_inv_launch<A, B>(nb13, sh13, c->stream, xi, y1, y2, c->tw[1])
-  TPX_FOUR_STEP_SWITCH(g.nx, L_XYI)
+  if (g.nx == 512) xy_inv_rp_launch(nb13, sh13, c->stream, xi, y1, y2, c->tw[1]);
+  else { TPX_FOUR_STEP_SWITCH(g.nx, L_XYI) }
 #undef L_XYI
   TPX_LAUNCH_CHECK();
   return nb13;
@@ -1792,7 +1975,7 @@ void launch_poisson_iteration_on(tpx_ctx *c, const double *rho_new, double *P, c
 void launch_coef_iteration(tpx_ctx *c, const double *const cf[3], double *P, const double *rhs, double *res) {
   const Geo &g = c->g;
   int r1, r2, y1, y2, z1, z2;
-  if (three_pass_shape(c, r1, r2, y1, y2, z1, z2)) {
+  if (three_pass_shape(c, r1, r2, y1, y2, z1, z2, aligned16({cf[0], cf[1], cf[2], P, rhs}))) {
     const double *done = c->iter_ctl.first ? nullptr : c->scal + SC_DONE;
     timing_begin(c, TPX_K_FFT);
     XArgs xa{g, P, nullptr, rhs, c->scal, c->spec[0], c->tw[0], (double)g.n, done, nullptr};
