@@ -144,6 +144,68 @@ __device__ void lds_fft(double2 *buf, int n, int lines, const double2 *__restric
   }
 }
 
+// The loop test of a solve whose iterations are launched one after another
+// (poisson.cpp:391-462: go on while count < Iteration and max |dp| > epsilon).
+// Pass 3 folds its blocks' maxima into 16 slots, a cache line each, with atomic
+// maxima that nobody waits for (non-negative doubles order as their bits; the
+// maximum does not depend on the order).  The first 16 threads of the next
+// iteration's pass 1 pick the slots up beside their own work and write the
+// test's outcome down, which passes 2 and 3 of that iteration and all later
+// ones read: a pass 1 that turns out to have been one too many has only written
+// the spectrum.  A kernel over the block maxima after every iteration cost 3-5
+// us of an iteration of 20 at 32^3 and 63 at 128^3; evaluated by every block of
+// pass 1 before its work, the test cost that pass 1-3 us.
+constexpr int kDpSlots = 16, kDpSet = kDpSlots * 8;  // slots of a set; 8-byte values of a set
+struct LoopState {
+  uint64_t *slots = nullptr;  // two sets: iteration i uses set i % 2 (null: no loop test here)
+  double *scal = nullptr;
+  uint64_t *host = nullptr;   // pinned memory that receives the loop state (null: none)
+  double epsilon = 0.0;
+  int index = 0;              // iterations before this one
+  int iteration = 0;
+  uint32_t epoch = 0;
+  __device__ void to_global() {
+    slots = gptr(slots);
+    scal = gptr(scal);
+    host = gptr(host);
+  }
+};
+
+// the slot of the last iteration that this thread picks up (the first 16
+// threads of the launch); loop_note takes it
+__device__ __forceinline__ uint64_t loop_peek(const LoopState &s) {
+  if (!s.slots || blockIdx.x != 0 || threadIdx.x >= kDpSlots || s.index == 0) return 0;
+  return s.slots[((s.index - 1) & 1) * kDpSet + threadIdx.x * 8];
+}
+
+// the outcome of the loop test before iteration s.index
+__device__ __forceinline__ void loop_note(const LoopState &s, uint64_t m) {
+  if (!s.slots || blockIdx.x != 0 || threadIdx.x >= kDpSlots) return;
+  if (s.index == 0) {
+    s.slots[threadIdx.x * 8] = 0;
+    if (threadIdx.x == 0) {
+      s.scal[SC_ITERS] = 0.0;
+      s.scal[SC_DONE] = 0.0;
+    }
+    return;
+  }
+#pragma unroll
+  for (int o = kDpSlots / 2; o > 0; o >>= 1) {
+    const uint64_t other = (uint64_t)__shfl_xor((unsigned long long)m, o, kDpSlots);
+    m = other > m ? other : m;
+  }
+  if (threadIdx.x == 0 && s.scal[SC_DONE] == 0.0) {
+    const double err = __longlong_as_double((long long)m);
+    const bool more = s.index < s.iteration && err > s.epsilon;
+    s.scal[SC_MAX_DP] = err;
+    s.scal[SC_ITERS] = (double)s.index;
+    s.scal[SC_DONE] = more ? 0.0 : 1.0;
+    if (s.host)  // the host reads the loop state from its own memory as the solve goes
+      __hip_atomic_store(s.host, ((uint64_t)s.epoch << 32) | ((uint64_t)s.index << 1) | (more ? 0 : 1), __ATOMIC_RELEASE,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 struct XArgs {
   Geo g;
   const double *P;
@@ -161,6 +223,7 @@ struct XArgs {
                                // residual (P, rho, rhs unread)
   const double *cf[3] = {};    // three-pass form, its own kernel instance: the caller's face
                                // coefficient in the place of 1 / Rho_face (rho unread, RHS as given)
+  LoopState loop;              // three-pass form: the loop test (slots null: `done` says it all)
   __device__ void to_global() {
     P = gptr(P);
     rho = gptr(rho);
@@ -172,6 +235,7 @@ struct XArgs {
     res = gptr(res);
     in = gptr(in);
     for (auto &q : cf) q = gptr(q);
+    loop.to_global();
   }
 };
 
@@ -345,6 +409,7 @@ struct XInvArgs {
   const double *done;
   int overwrite = 0;  // three-pass form: P = dp (P unread, its own kernel instance) instead of P += dp
   double *Pout = nullptr;  // non-null: P + dp is written here and P is left as it was
+  uint64_t *slots = nullptr;  // three-pass form: max |dp| goes into this set of slots, not into partials
   __device__ void to_global() {
     P = gptr(P);
     spec = gptr(spec);
@@ -352,6 +417,12 @@ struct XInvArgs {
     partials = gptr(partials);
     done = gptr(done);
     Pout = gptr(Pout);
+    slots = gptr(slots);
+  }
+  // a block's max |dp|
+  __device__ __forceinline__ void block_max_dp(unsigned blk, double v) const {
+    if (slots) atomicMax((unsigned long long *)&slots[(blk % kDpSlots) * 8], (unsigned long long)__double_as_longlong(v));
+    else partials[blk] = v;
   }
 };
 
@@ -928,6 +999,7 @@ struct k_xy_fwd {
   static constexpr int kBounds = 256;
   static __device__ __forceinline__ void run(const XArgs &a, int Y1, const double2 *__restrict__ twy) {
   if (a.done && *a.done != 0.0) return;  // the solve has converged
+  const uint64_t dp_slot = loop_peek(a.loop);
   extern __shared__ double ldsd[];
   constexpr int n = R1 * R2, P = R1 + 1, SP = Y2 + 1;  // padded rows of the x exchange and of the kx columns
   const Geo &g = a.g;
@@ -997,6 +1069,7 @@ struct k_xy_fwd {
 #pragma unroll
     for (int k2 = 0; k2 < Y2; ++k2) dst[k2 * ks] = w[k2];
   }
+  loop_note(a.loop, dp_slot);
 }
 };
 
@@ -1011,8 +1084,9 @@ struct k_yz_pass {
                                                  const double *__restrict__ lamx,
                                                  const double *__restrict__ lamy,
                                                  const double *__restrict__ lamz,
-                                                 const double *__restrict__ done) {
+                                                 const double *__restrict__ done, uint64_t *clear) {
   if (done && *done != 0.0) return;  // the solve has converged
+  if (clear && blockIdx.x == 0 && threadIdx.x < kDpSlots) clear[threadIdx.x * 8] = 0;  // the next iteration's slots
   extern __shared__ double2 L[];
   constexpr int nz = Z1 * Z2, NE = nz * Y1, RS = nz + nz / 16;
   auto pad = [](int e) { return e + (e >> 4); };  // one spare slot every 16: fewer bank conflicts
@@ -1285,6 +1359,7 @@ struct k_xy_fwd_rp {
   static constexpr int kBounds = 256;
   static __device__ __forceinline__ void run(const XArgs &a, int Y1, const double2 *__restrict__ twy) {
     if (a.done && *a.done != 0.0) return;  // the solve has converged
+    const uint64_t dp_slot = loop_peek(a.loop);
     extern __shared__ double ldsd[];
     constexpr int R1 = 16, M = R1 * R2H, P = R1 + 1, SP = Y2 + 1;
     const Geo &g = a.g;
@@ -1353,6 +1428,7 @@ struct k_xy_fwd_rp {
 #pragma unroll
       for (int k2 = 0; k2 < Y2; ++k2) dst[k2 * ks] = w[k2];
     }
+    loop_note(a.loop, dp_slot);
   }
 };
 
@@ -1453,7 +1529,7 @@ struct k_xy_inv_rp {
       if ((int)threadIdx.x < s) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + s]);
       __syncthreads();
     }
-    if (threadIdx.x == 0) a.partials[blk] = red[0];
+    if (threadIdx.x == 0) a.block_max_dp(blk, red[0]);
   }
 };
 
@@ -1555,7 +1631,7 @@ struct k_xy_inv {
     if ((int)threadIdx.x < s) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + s]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) a.partials[blk] = red[0];
+  if (threadIdx.x == 0) a.block_max_dp(blk, red[0]);
 }
 };
 
@@ -1609,6 +1685,12 @@ struct k_finish_iter {
                          __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
+};
+
+// the loop test after the last iteration launched so far (see LoopState)
+struct k_loop_check {
+  static constexpr int kBounds = 64;
+  static __device__ __forceinline__ void run(const LoopState &s) { loop_note(s, loop_peek(s)); }
 };
 
 // Start of a solve: no iteration yet, err = 100 (poisson.cpp:391-396)
@@ -1759,10 +1841,10 @@ size_t yz_shared_bytes(int y1, int nz) {
 }
 template <int Z1, int Z2>
 void yz_launch(unsigned nb, size_t sh, hipStream_t st, double2 *spec, int mxh, int Y1, int Y2, const tpx_ctx *c,
-               const double *done) {
+               const double *done, uint64_t *clear) {
 #define L_YZ1(Y)                                                                                                  \
   tpx_launch<k_yz_pass<Y, Z1, Z2>>(nb, k_yz_pass<Y, Z1, Z2>::kBounds, sh, st, spec, mxh, Y2, c->tw[2], c->lam[0], \
-                                   c->lam[1], c->lam[2], done)
+                                   c->lam[1], c->lam[2], done, clear)
   switch (Y1) {
     case 4: L_YZ1(4); break;
     case 8: L_YZ1(8); break;
@@ -1777,6 +1859,27 @@ void yz_launch(unsigned nb, size_t sh, hipStream_t st, double2 *spec, int mxh, i
 void launch_solve_state(tpx_ctx *c, double *dst) {
   tpx_launch<k_solve_state>(1, 64, 0, c->stream, (const double *)c->scal, dst);
   TPX_LAUNCH_CHECK();
+}
+
+// the loop state of the iteration being launched, or none (its own finish kernel)
+static LoopState loop_of(tpx_ctx *c, int index) {
+  LoopState s;
+  if (index < 0) return s;
+  s.slots = c->dp_slots;
+  s.scal = c->scal;
+  s.host = c->iter_ctl.host;
+  s.epsilon = c->p.epsilon;
+  s.index = index;
+  s.iteration = c->Iteration;
+  s.epoch = c->iter_ctl.epoch;
+  return s;
+}
+
+void launch_loop_check(tpx_ctx *c) {
+  if (c->iter_ctl.pending == 0) return;
+  tpx_launch<k_loop_check>(1, 64, 0, c->stream, loop_of(c, c->iter_ctl.pending));
+  TPX_LAUNCH_CHECK();
+  c->iter_ctl.pending = 0;
 }
 
 void launch_solve_begin(tpx_ctx *c) {
@@ -1858,7 +1961,8 @@ unsigned three_pass_launch(tpx_ctx *c, const XArgs &xa, const XInvArgs &xi, cons
   timing_begin(c, TPX_K_FFT_YZ);
   const unsigned nb2 = (unsigned)(mxh * y2);
   const size_t sh2 = yz_shared_bytes(y1, g.nz);
-#define L_YZ(A, B) yz_launch<A, B>(nb2, sh2, c->stream, c->spec[0], mxh, y1, y2, c, done)
+  uint64_t *clear = xa.loop.slots ? xa.loop.slots + ((xa.loop.index + 1) & 1) * kDpSet : nullptr;
+#define L_YZ(A, B) yz_launch<A, B>(nb2, sh2, c->stream, c->spec[0], mxh, y1, y2, c, done, clear)
   if (g.nz == 512) L_YZ(16, 32);
   else { TPX_FOUR_STEP_SWITCH(g.nz, L_YZ) }
 #undef L_YZ
@@ -1871,6 +1975,23 @@ unsigned three_pass_launch(tpx_ctx *c, const XArgs &xa, const XInvArgs &xi, cons
 #undef L_XYI
   TPX_LAUNCH_CHECK();
   return nb13;
+}
+
+// One iteration in the three-pass form with its loop test: through the slots
+// where the solve is launched iteration by iteration on the context's scalars,
+// else (a batch's captured iteration, which does not know its number) by a
+// kernel over the block maxima.
+static void three_pass_iteration(tpx_ctx *c, XArgs &xa, XInvArgs &xi, const double *done, int r1, int r2, int y1, int y2,
+                                 double *scal) {
+  const int index = scal == c->scal ? c->iter_ctl.index : -1;
+  xa.loop = loop_of(c, index);
+  if (index >= 0) xi.slots = c->dp_slots + (index & 1) * kDpSet;
+  const unsigned nb13 = three_pass_launch(c, xa, xi, done, r1, r2, y1, y2);
+  if (index >= 0) c->iter_ctl.pending = index + 1;
+  else
+    tpx_launch<k_finish_iter>(1, 1024, 0, c->stream, c->partials, nb13, scal, c->Iteration, c->p.epsilon, c->iter_ctl);
+  TPX_LAUNCH_CHECK();
+  timing_end(c, TPX_K_FFT_INV);
 }
 
 void launch_poisson_iteration_on(tpx_ctx *c, const double *rho_new, double *P, const double *rhs, double *scal,
@@ -1891,10 +2012,7 @@ void launch_poisson_iteration_on(tpx_ctx *c, const double *rho_new, double *P, c
   // the three-pass form forms the residual itself from rho; a precomputed
   // residual goes through the five-pass kernels
   if (!res && three_pass_shape(c, r1, r2, y1, y2, z1, z2)) {
-    const unsigned nb13 = three_pass_launch(c, xa, xi, done, r1, r2, y1, y2);
-    tpx_launch<k_finish_iter>(1, 1024, 0, c->stream, c->partials, nb13, scal, c->Iteration, c->p.epsilon, c->iter_ctl);
-    TPX_LAUNCH_CHECK();
-    timing_end(c, TPX_K_FFT_INV);
+    three_pass_iteration(c, xa, xi, done, r1, r2, y1, y2, scal);
     return;
   }
   const int cx = x4 ? 128 / r1 : lines_per_block(g.nx);
@@ -1986,11 +2104,8 @@ void launch_coef_iteration(tpx_ctx *c, const double *const cf[3], double *P, con
     timing_begin(c, TPX_K_FFT);
     XArgs xa{g, P, nullptr, rhs, c->scal, c->spec[0], c->tw[0], (double)g.n, done, nullptr};
     for (int d = 0; d < 3; ++d) xa.cf[d] = cf[d];
-    const XInvArgs xi{g, P, c->spec[0], c->tw[0], c->partials, -1.0 / (double)g.n, done};
-    const unsigned nb13 = three_pass_launch(c, xa, xi, done, r1, r2, y1, y2);
-    tpx_launch<k_finish_iter>(1, 1024, 0, c->stream, c->partials, nb13, c->scal, c->Iteration, c->p.epsilon, c->iter_ctl);
-    TPX_LAUNCH_CHECK();
-    timing_end(c, TPX_K_FFT_INV);
+    XInvArgs xi{g, P, c->spec[0], c->tw[0], c->partials, -1.0 / (double)g.n, done};
+    three_pass_iteration(c, xa, xi, done, r1, r2, y1, y2, c->scal);
     return;
   }
   launch_residual_coef(c, cf, P, rhs, res);

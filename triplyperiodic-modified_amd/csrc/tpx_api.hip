@@ -458,7 +458,7 @@ int solve_loop(tpx_ctx *c, int guess, const std::function<void(int)> &iterate) {
   struct Running {  // the iterations of this solve report to the host
     tpx_ctx *c;
     explicit Running(tpx_ctx *ctx) : c(ctx) {
-      c->iter_ctl = {1, ++c->solve_epoch, c->h_iter};
+      c->iter_ctl = {1, ++c->solve_epoch, c->h_iter, 0, 0};
     }
     ~Running() { c->iter_ctl = {}; }
   } running(c);
@@ -467,7 +467,9 @@ int solve_loop(tpx_ctx *c, int guess, const std::function<void(int)> &iterate) {
     for (; n > 0 && queued < c->Iteration; --n) {
       iterate(queued++);
       c->iter_ctl.first = 0;
+      ++c->iter_ctl.index;
     }
+    launch_loop_check(c);
   };
   queue(std::max(1, guess));
   bool stopped = false;
@@ -730,7 +732,7 @@ void release(tpx_ctx *c) {
   for (auto &p : c->spec) f(p);
   for (auto &p : c->lam) f(p);
   for (auto &p : c->tw) f(p);
-  f(c->scal); f(c->partials); f(c->scan_tmp); f(c->st_part);
+  f(c->scal); f(c->dp_slots); f(c->partials); f(c->scan_tmp); f(c->st_part);
   for (auto &p : c->ps) f(p);
   adjoint_free(c->adj);
   tape_give_back(c->adj, 0);
@@ -887,6 +889,7 @@ int tpx_create(const tpx_params *p, int64_t np_capacity, tpx_ctx **out) {
     if (np_capacity > 0) dalloc(&c->dep_tmp, 3 * n);
     for (auto &f : c->S) dalloc(&f, n);
     dalloc(&c->scal, SC_COUNT);
+    if (hipMalloc(&c->dp_slots, sizeof(uint64_t) * 256) != hipSuccess) throw std::bad_alloc();
     // one partial per 256-cell block or per x-row, whichever is more
     c->n_partials = std::max((long)grid1d(g.n, 256), (long)g.ny * g.nz) + 1024;
     dalloc(&c->partials, 3 * (size_t)c->n_partials);
@@ -1804,6 +1807,10 @@ void gas_substeps(tpx_ctx *c, int s, GasSubstep sub[4], bool segment) {
     g.iters = t.iters[q];
     if (g.iters == 0) launch_solve_begin(c);
     if (segment) t.p_first[q] = used;
+    struct Numbered {  // the replayed iterations evaluate the loop test as the run's did
+      tpx_ctx *c;
+      ~Numbered() { c->iter_ctl = {}; }
+    } numbered{c};
     for (int it = 0; it < g.iters; ++it) {
       double *buf = pcap_slot(t, used++, n);
       if (!buf) throw std::bad_alloc();
@@ -1812,9 +1819,10 @@ void gas_substeps(tpx_ctx *c, int s, GasSubstep sub[4], bool segment) {
       double *out = c->P;
       if (it + 1 < g.iters && !(out = pcap_slot(t, used, n))) throw std::bad_alloc();
       c->iter_ctl.first = it == 0;
+      c->iter_ctl.index = it;
       launch_poisson_iteration_on(c, c->rho[c->rho_new], buf, g.rhs, c->scal, nullptr, SC_SUM_RHS, out);
-      c->iter_ctl.first = 0;
     }
+    launch_loop_check(c);
     launch_copy(c, t.iters_seen + (long)s * 4 + rk, c->scal + SC_ITERS, 1);
     do_update_ru_wp(c, rk, rk == 3, true);
     c->rho_int = c->rho_new;  // the gas half of TimeAdvance_RK4

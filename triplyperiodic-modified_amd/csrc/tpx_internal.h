@@ -252,12 +252,17 @@ struct HostStage {
 
 // How a Poisson iteration takes part in its solve's loop: `first` iterations
 // run without reading the loop test (and restart the count), and `host`, if
-// set, is pinned memory that receives epoch << 32 | iterations << 1 | stopped
-// after each one.
+// set, is pinned memory that receives epoch << 32 | iterations << 1 | stopped.
+// With index >= 0 (the iteration's number in its solve) the three-pass form
+// leaves max |dp| in the context's slots and the next pass 1 evaluates the loop
+// test; `pending` is then the iterations whose test a launch_loop_check still
+// owes.
 struct IterCtl {
   int first = 0;
   uint32_t epoch = 0;
   uint64_t *host = nullptr;
+  int index = -1;
+  int pending = 0;
   __device__ void to_global() { host = gptr(host); }
 };
 
@@ -288,6 +293,7 @@ struct tpx_ctx {
   int vec_guess[4] = {2, 2, 2, 2}; // and for the passive vector's
   tpx::IterCtl iter_ctl;           // of the iteration being launched
   uint64_t *h_iter = nullptr;      // pinned, coherent: the loop state of the running solve
+  uint64_t *dp_slots = nullptr;    // max |dp| of an iteration, spread over cache lines; two sets in turn
   uint32_t solve_epoch = 0;
   hipStream_t stream = nullptr;
   int device = 0;
@@ -405,6 +411,9 @@ void launch_track(tpx_ctx *c, int stride, int count, double *out);
 // grid::Update_Passive_Scalar (k_grid.hip) and the sum of its source
 void launch_passive_scalar(tpx_ctx *c, const Coef &k, const double *const ru_int[3], const double *rho_int);
 void launch_passive_scalar_source_sum(tpx_ctx *c);
+// evaluates the loop test of the iterations launched so far where the next
+// iteration's pass 1 would (nothing where each iteration evaluates its own)
+void launch_loop_check(tpx_ctx *c);
 // resets the device-side iteration count and loop test of a solve
 void launch_solve_begin(tpx_ctx *c);
 // copies the solve's iteration count and stopped flag to dst[0..1] (device)
