@@ -983,16 +983,26 @@ struct k_zpass4 {
 //   pass 3, block (z, t):   inverse y step A (twiddle W_ny^{-t k2}, DFT over
 //                           k2 back to m) for every kx, inverse x transform
 //                           of the Y2 rows, P += dp, block max |dp|.
-// Between the passes the spectrum is stored as
-//   S[(k2 mxh + kx) CS + z Y1 + t],   CS = nz Y1 + 8,
-// so a pass-2 block reads and writes one contiguous nz Y1 run, and the Y1
-// blocks (z, 0..Y1-1) of passes 1 and 3, which run next to each other on one
-// XCD, share every 256-byte run of it.  In passes 1 and 3 the lanes of a wave
-// take consecutive kx, 16 nz Y1 + 128 bytes apart: the 128 spare bytes per
-// run spread those accesses over the L2 channels (at a stride of a power of
-// two they would all queue on one).  Two passes over the spectrum fewer than
-// the five-pass form.
-constexpr int kRunPad = 8;  // spare complex values after each nz Y1 run
+// Between the passes the spectrum is stored in groups of two kx,
+//   S[(k2 G + kx / 2) CS + 2 (z Y1 + t) + kx % 2],   CS = 2 nz Y1 + 8,
+// G = groups_of(mxh), so two pass-2 blocks beside each other on one XCD read
+// and write one contiguous run of 2 nz Y1, and the Y1 blocks (z, 0..Y1-1) of
+// passes 1 and 3, which run next to each other on one XCD, share every line of
+// it.  In passes 1 and 3 the lanes of a wave take consecutive kx, so a store or
+// load of 64 lanes touches 32 pieces of 32 bytes, CS apart: the 128 spare bytes
+// per run spread those over the L2 channels (at a stride of a power of two they
+// would all queue on one).  Those requests, about one a nanosecond on each of
+// the 128 channels, bound both passes where the spectrum stays in the caches.
+// One kx a run (64 pieces of 16 bytes) measured 24.6 + 17.8 + 15.9 us an
+// iteration at 128^3 and 43.7 + 23.1 + 29.7 at 512 x 64 x 128; two 21.5 + 18.3 +
+// 14.2 and 36.4 + 24.3 + 24.5; four 21.3 + 19.8 + 14.0 and 34.6 + 29.1 + 25.0
+// (pass 2 then takes 16 bytes of every 64); 64^3 and below and 256^3 are level.
+// A pass-2 block for both kx of a run needs twice the waves and LDS at once and
+// is slower (26.5 against 18.5 us at 128^3).  Two passes over the spectrum
+// fewer than the five-pass form.
+constexpr int kRunPad = 8;  // spare complex values after each run
+constexpr int kGroup = 2;   // kx values side by side in a run
+__host__ __device__ constexpr int groups_of(int mxh) { return (mxh + kGroup - 1) / kGroup; }
 // ---------------------------------------------------------------------------
 template <int R1, int R2, int Y2, bool Coef = false>
 struct k_xy_fwd {
@@ -1058,14 +1068,14 @@ struct k_xy_fwd {
   }
   __syncthreads();
   // y step A for every kx
-  const long cs = (long)g.nz * Y1 + kRunPad;
-  const long ks = cs * mxh;  // distance between consecutive k2
+  const long cs = kGroup * (long)g.nz * Y1 + kRunPad;
+  const long ks = cs * groups_of(mxh);  // distance between consecutive k2
   for (int kx = threadIdx.x; kx < mxh; kx += block_dim_x()) {
     double2 w[Y2];
 #pragma unroll
     for (int m = 0; m < Y2; ++m) w[m] = S[kx * SP + m];
     step_a<Y2, false>(w, t, twy);
-    double2 *dst = a.spec + kx * cs + z * Y1 + t;
+    double2 *dst = a.spec + kx / kGroup * cs + kGroup * (z * Y1 + t) + kx % kGroup;
 #pragma unroll
     for (int k2 = 0; k2 < Y2; ++k2) dst[k2 * ks] = w[k2];
   }
@@ -1105,7 +1115,7 @@ struct k_yz_pass {
   auto pad = [](int e) { return e + (e >> 4); };  // one spare slot every 16: fewer bank conflicts
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
   const int k2 = (int)(blk / (unsigned)mxh), kx = (int)(blk % (unsigned)mxh);
-  // element (z, t) at z Y1 + t.  The run and the tables are read through
+  // element (z, t) at kGroup (z Y1 + t) of the group's run.  The run and the tables are read through
   // global-address-space pointers: in the batched launch the arguments come
   // from a table in memory as generic pointers, whose flat loads also count
   // against the LDS wait counter (and the register staging below went
@@ -1114,7 +1124,7 @@ struct k_yz_pass {
   typedef __attribute__((address_space(1))) dv2 gdv2;
   typedef __attribute__((address_space(1))) const dv2 gcdv2;
   typedef __attribute__((address_space(1))) const double gcdouble;
-  gdv2 *base = (gdv2 *)(spec + (long)blk * (NE + kRunPad));
+  gdv2 *base = (gdv2 *)(spec + (long)(k2 * groups_of(mxh) + kx / kGroup) * (kGroup * NE + kRunPad) + kx % kGroup);
   const int tid = threadIdx.x;
   // the z twiddles and lambda_z beside the run (yz_shared_bytes), copied in
   // with it: the transform stages then wait on LDS for them, not on global
@@ -1138,7 +1148,7 @@ struct k_yz_pass {
     for (int u = 0; u < NU; ++u) {
       const int e = tid + u * kBounds;
       if (NE % kBounds == 0 || e < NE) {
-        const dv2 q = base[e];
+        const dv2 q = base[kGroup * e];
         r[u] = make_double2(q.x, q.y);
       }
     }
@@ -1255,7 +1265,7 @@ struct k_yz_pass {
     const int e = t3 + u * kBounds;
     if (NE % kBounds == 0 || e < NE) {
       const double2 q = L[pad(e)];
-      base[e] = dv2{q.x, q.y};
+      base[kGroup * e] = dv2{q.x, q.y};
     }
   }
 }
@@ -1430,8 +1440,8 @@ struct k_xy_fwd_rp {
       for (int k1 = 0; k1 < R1; ++k1) S[(k2x + R2H * k1) * SP + cb] = u[k1];
     }
     __syncthreads();
-    const long cs = (long)g.nz * Y1 + kRunPad;
-    const long ks = cs * mxh;
+    const long cs = kGroup * (long)g.nz * Y1 + kRunPad;
+    const long ks = cs * groups_of(mxh);
     for (int kx = threadIdx.x; kx < mxh; kx += block_dim_x()) {
       const double2 wn = a.tw[kx];  // W_2M^kx
       const int ka = kx & (M - 1), kb = (M - kx) & (M - 1);
@@ -1445,7 +1455,7 @@ struct k_xy_fwd_rp {
         w[m] = cadd(E, cmul(wn, O));
       }
       step_a<Y2, false>(w, t, twy);
-      double2 *dst = a.spec + kx * cs + z * Y1 + t;
+      double2 *dst = a.spec + kx / kGroup * cs + kGroup * (z * Y1 + t) + kx % kGroup;
 #pragma unroll
       for (int k2 = 0; k2 < Y2; ++k2) dst[k2 * ks] = w[k2];
     }
@@ -1474,10 +1484,10 @@ struct k_xy_inv_rp {
     const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
     const int t = (int)(blk % (unsigned)Y1), z = (int)(blk / (unsigned)Y1);
     double2 *S = reinterpret_cast<double2 *>(ldsd);  // S[kx SP + row]
-    const long cs = (long)g.nz * Y1 + kRunPad;
-    const long ks = cs * mxh;
+    const long cs = kGroup * (long)g.nz * Y1 + kRunPad;
+    const long ks = cs * groups_of(mxh);
     for (int kx = threadIdx.x; kx < mxh; kx += block_dim_x()) {
-      const double2 *src = a.spec + kx * cs + z * Y1 + t;
+      const double2 *src = a.spec + kx / kGroup * cs + kGroup * (z * Y1 + t) + kx % kGroup;
       double2 w[Y2];
 #pragma unroll
       for (int k2 = 0; k2 < Y2; ++k2) {
@@ -1568,10 +1578,10 @@ struct k_xy_inv {
   const int t = (int)(blk % (unsigned)Y1), z = (int)(blk / (unsigned)Y1);
   double2 *S = reinterpret_cast<double2 *>(ldsd);  // S[kx SP + row]
   // inverse y step A for every kx: row m is y = t + Y1 m
-  const long cs = (long)g.nz * Y1 + kRunPad;
-  const long ks = cs * mxh;
+  const long cs = kGroup * (long)g.nz * Y1 + kRunPad;
+  const long ks = cs * groups_of(mxh);
   for (int kx = threadIdx.x; kx < mxh; kx += block_dim_x()) {
-    const double2 *src = a.spec + kx * cs + z * Y1 + t;
+    const double2 *src = a.spec + kx / kGroup * cs + kGroup * (z * Y1 + t) + kx % kGroup;
     double2 w[Y2];
 #pragma unroll
     for (int k2 = 0; k2 < Y2; ++k2) {
@@ -1770,8 +1780,8 @@ int fft_setup(tpx_ctx *c) {
     if (hipMemcpy(c->lam[a], lam.data(), sizeof(double) * lam.size(), hipMemcpyHostToDevice) != hipSuccess) return TPX_E_HIP;
   }
   long mxh = g.nx / 2 + 1;
-  // the three-pass layout leaves kRunPad spare values after each of its mxh Y2 runs
-  if (hipMalloc(&c->spec[0], sizeof(double2) * mxh * ((long)g.ny * g.nz + 16 * kRunPad)) != hipSuccess)
+  // the three-pass layout leaves kRunPad spare values after each of its groups_of(mxh) Y2 runs
+  if (hipMalloc(&c->spec[0], sizeof(double2) * kGroup * groups_of(mxh) * ((long)g.ny * g.nz + 16 * kRunPad)) != hipSuccess)
     return TPX_E_OOM;
   return TPX_OK;
 }
