@@ -1385,21 +1385,33 @@ __device__ __forceinline__ void row_residuals_pairs_coef(const XArgs &a, const I
 
 // pass 1, packed: residual rows, the M-point x transform, the half spectrum
 // recovered on the way out of LDS, y step A
+// With 8 rows a t (128 lanes) and x lengths from 128 on, a block takes two
+// neighbouring t, each with 128 lanes and its own part of the LDS: four
+// adjacent lanes of the store then write 64 bytes, two kx of both t, and the
+// rows the two t share are read by one CU (37.4 to 34.0 us a pass at
+// 512 x 64 x 128, 17.0 to 15.9 at 256 x 64 x 64, 22.1 to 21.6 at 128^3).  At x
+// length 64 and with 4 rows it measured level or slower, and with 16 rows the
+// block would be 512 lanes and one on a CU.
 template <int R2H, int Y2, bool Coef = false>
 struct k_xy_fwd_rp {
-  static constexpr int kBounds = 256;
+  static constexpr int kBounds = 256, T = R2H >= 4 && Y2 == 8 ? 2 : 1, H = Y2 * 16;
+  // doubles of one row set: an odd number of 64 bytes, so that the four lanes of
+  // a store, which read two kx of both sets, read four banks
+  static constexpr int kHalf = (std::max(Y2 * R2H * 17, 16 * R2H * (Y2 + 1) * 2) + 15) / 16 * 16 + 8;
   static __device__ __forceinline__ void run(const XArgs &a, int Y1, const double2 *__restrict__ twy) {
     if (a.done && *a.done != 0.0) return;  // the solve has converged
     const uint64_t dp_slot = loop_peek(a.loop);
-    extern __shared__ double ldsd[];
+    extern __shared__ double lds_all[];
     constexpr int R1 = 16, M = R1 * R2H, P = R1 + 1, SP = Y2 + 1;
     const Geo &g = a.g;
     const int mxh = M + 1;
     Ix ix{g.nx - 1, g.ny - 1, g.nz - 1, g.nx, g.nxy};
     const double mean = a.scal[SC_SUM_RHS] / a.ncell;
     const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
-    const int t = (int)(blk % (unsigned)Y1), z = (int)(blk / (unsigned)Y1);
-    const int ta = threadIdx.x % R1, ca = threadIdx.x / R1;
+    const int t0 = T * (int)(blk % (unsigned)(Y1 / T)), z = (int)(blk / (unsigned)(Y1 / T));
+    const int h = threadIdx.x / H, lane = threadIdx.x % H, t = t0 + h;
+    double *ldsd = lds_all + h * kHalf;
+    const int ta = lane % R1, ca = lane / R1;
     double2 v[R2H];
     if constexpr (Coef) {
       row_residuals_pairs_coef<R2H>(a, ix, ta, t + Y1 * ca, z, v);
@@ -1414,8 +1426,8 @@ struct k_xy_fwd_rp {
     RegDft<R2H, false>::run(v);
 #pragma unroll
     for (int k2 = 1; k2 < R2H; ++k2) v[k2] = cmul(v[k2], a.tw[2 * ta * k2]);
-    const bool b_item = (int)threadIdx.x < Y2 * R2H;
-    const int k2x = threadIdx.x % R2H, cb = threadIdx.x / R2H;
+    const bool b_item = lane < Y2 * R2H;
+    const int k2x = lane % R2H, cb = lane / R2H;
     double2 u[R1];
 #pragma unroll
     for (int q = 0; q < R2H; ++q) ldsd[(ca * R2H + q) * P + ta] = v[q].x;
@@ -1442,20 +1454,23 @@ struct k_xy_fwd_rp {
     __syncthreads();
     const long cs = kGroup * (long)g.nz * Y1 + kRunPad;
     const long ks = cs * groups_of(mxh);
-    for (int kx = threadIdx.x; kx < mxh; kx += block_dim_x()) {
+    for (int e = threadIdx.x; e < (T > 1 ? T * kGroup * groups_of(mxh) : mxh); e += block_dim_x()) {
+      const int kx = e / (kGroup * T) * kGroup + e % kGroup, he = e / kGroup % T;
+      if (T > 1 && kx >= mxh) continue;
+      const double2 *Se = reinterpret_cast<const double2 *>(lds_all + he * kHalf);
       const double2 wn = a.tw[kx];  // W_2M^kx
       const int ka = kx & (M - 1), kb = (M - kx) & (M - 1);
       double2 w[Y2];
 #pragma unroll
       for (int m = 0; m < Y2; ++m) {
-        const double2 A = S[ka * SP + m], B = S[kb * SP + m];
+        const double2 A = Se[ka * SP + m], B = Se[kb * SP + m];
         const double2 E = make_double2((A.x + B.x) * 0.5, (A.y - B.y) * 0.5);   // (A + conj B) / 2
         const double2 D = make_double2((A.x - B.x) * 0.5, (A.y + B.y) * 0.5);   // (A - conj B) / 2
         const double2 O = make_double2(D.y, -D.x);                              // D / i
         w[m] = cadd(E, cmul(wn, O));
       }
-      step_a<Y2, false>(w, t, twy);
-      double2 *dst = a.spec + kx / kGroup * cs + kGroup * (z * Y1 + t) + kx % kGroup;
+      step_a<Y2, false>(w, t0 + he, twy);
+      double2 *dst = a.spec + kx / kGroup * cs + kGroup * (z * Y1 + t0 + he) + kx % kGroup;
 #pragma unroll
       for (int k2 = 0; k2 < Y2; ++k2) dst[k2 * ks] = w[k2];
     }
@@ -1503,7 +1518,9 @@ struct k_xy_inv_rp {
       for (int m = 0; m < Y2; ++m) S[kx * SP + m] = w[m];
     }
     __syncthreads();
-    const int tx = threadIdx.x % R1, c = threadIdx.x / R1;
+    // the block is these Y2 R1 lanes, as in k_xy_inv below
+    const int lane = threadIdx.x % (Y2 * R1);
+    const int tx = lane % R1, c = lane / R1;
     double2 v[R2H];
 #pragma unroll
     for (int m = 0; m < R2H; ++m) {
@@ -1523,8 +1540,8 @@ struct k_xy_inv_rp {
       v[k2] = cmul(v[k2], w);
     }
     __syncthreads();  // S is reused by the exchange
-    const bool b_item = (int)threadIdx.x < Y2 * R2H;
-    const int k2x = threadIdx.x % R2H, cb = threadIdx.x / R2H;
+    const bool b_item = lane < Y2 * R2H;
+    const int k2x = lane % R2H, cb = lane / R2H;
     double2 u[R1];
 #pragma unroll
     for (int q = 0; q < R2H; ++q) ldsd[(c * R2H + q) * P + tx] = v[q].x;
@@ -1598,7 +1615,10 @@ struct k_xy_inv {
   }
   __syncthreads();
   // inverse x: Hermitian extension of row c, step A over i = tx + R1 mm
-  const int tx = threadIdx.x % R1, c = threadIdx.x / R1;
+  // the block is these Y2 R1 lanes; written so, the compiler knows it and the
+  // 16 x 16 transform has no idle items to mask (85 to 75 us a pass at 256^3)
+  const int lane = threadIdx.x % (Y2 * R1);
+  const int tx = lane % R1, c = lane / R1;
   double2 v[R2];
 #pragma unroll
   for (int m = 0; m < R2; ++m) {
@@ -1615,8 +1635,8 @@ struct k_xy_inv {
   }
   step_a<R2, true>(v, tx, a.tw);
   __syncthreads();  // S is reused by the exchange
-  const bool b_item = (int)threadIdx.x < Y2 * R2;
-  const int k2x = threadIdx.x % R2, cb = threadIdx.x / R2;
+  const bool b_item = lane < Y2 * R2;
+  const int k2x = lane % R2, cb = lane / R2;
   double2 u[R1];
 #pragma unroll
   for (int q = 0; q < R2; ++q) ldsd[(c * R2 + q) * P + tx] = v[q].x;
@@ -1824,18 +1844,22 @@ void xy_fwd_launch(unsigned nb, size_t sh, hipStream_t st, const XArgs &xa, int 
   else xy_fwd_launch_t<R1, R2, false>(nb, sh, st, xa, Y1, Y2, twy);
 }
 // the packed forward form for x lengths 64, 128, 256 and 512 (R2H = 2, 4, 8, 16)
+template <class K>
+void xy_fwd_rp_start(hipStream_t st, int nz, const XArgs &xa, int Y1, const double2 *twy) {
+  tpx_launch<K>((unsigned)(nz * (Y1 / K::T)), K::T * K::H, sizeof(double) * K::T * K::kHalf, st, xa, Y1, twy);
+}
 template <int R2H, bool Coef>
-void xy_fwd_rp_launch_t(unsigned nb, size_t sh, hipStream_t st, const XArgs &xa, int Y1, int Y2, const double2 *twy) {
+void xy_fwd_rp_launch_t(hipStream_t st, int nz, const XArgs &xa, int Y1, int Y2, const double2 *twy) {
   switch (Y2) {
-    case 4: tpx_launch<k_xy_fwd_rp<R2H, 4, Coef>>(nb, 4 * 16, sh, st, xa, Y1, twy); break;
-    case 8: tpx_launch<k_xy_fwd_rp<R2H, 8, Coef>>(nb, 8 * 16, sh, st, xa, Y1, twy); break;
-    default: tpx_launch<k_xy_fwd_rp<R2H, 16, Coef>>(nb, 16 * 16, sh, st, xa, Y1, twy); break;
+    case 4: xy_fwd_rp_start<k_xy_fwd_rp<R2H, 4, Coef>>(st, nz, xa, Y1, twy); break;
+    case 8: xy_fwd_rp_start<k_xy_fwd_rp<R2H, 8, Coef>>(st, nz, xa, Y1, twy); break;
+    default: xy_fwd_rp_start<k_xy_fwd_rp<R2H, 16, Coef>>(st, nz, xa, Y1, twy); break;
   }
 }
 template <int R2H>
-void xy_fwd_rp_launch(unsigned nb, size_t sh, hipStream_t st, const XArgs &xa, int Y1, int Y2, const double2 *twy) {
-  if (xa.cf[0]) xy_fwd_rp_launch_t<R2H, true>(nb, sh, st, xa, Y1, Y2, twy);
-  else xy_fwd_rp_launch_t<R2H, false>(nb, sh, st, xa, Y1, Y2, twy);
+void xy_fwd_rp_launch(hipStream_t st, int nz, const XArgs &xa, int Y1, int Y2, const double2 *twy) {
+  if (xa.cf[0]) xy_fwd_rp_launch_t<R2H, true>(st, nz, xa, Y1, Y2, twy);
+  else xy_fwd_rp_launch_t<R2H, false>(st, nz, xa, Y1, Y2, twy);
 }
 template <int R1, int R2, bool Ow, bool Oop>
 void xy_inv_launch_t(unsigned nb, size_t sh, hipStream_t st, const XInvArgs &xi, int Y1, int Y2, const double2 *twy) {
@@ -1981,10 +2005,10 @@ unsigned three_pass_launch(tpx_ctx *c, const XArgs &xa, const XInvArgs &xi, cons
   bool packed = (g.nx == 64 || g.nx == 128 || g.nx == 256 || g.nx == 512) && c->x_packed;
   if (xa.cf[0]) packed = packed && aligned16({xa.cf[0], xa.cf[1], xa.cf[2], xa.P, xa.rhs});
 #define L_XYF(A, B) xy_fwd_launch<A, B>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1])
-  if (g.nx == 512) xy_fwd_rp_launch<16>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1]);
-  else if (packed && g.nx == 256) xy_fwd_rp_launch<8>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1]);
-  else if (packed && g.nx == 128) xy_fwd_rp_launch<4>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1]);
-  else if (packed) xy_fwd_rp_launch<2>(nb13, sh13, c->stream, xa, y1, y2, c->tw[1]);
+  if (g.nx == 512) xy_fwd_rp_launch<16>(c->stream, g.nz, xa, y1, y2, c->tw[1]);
+  else if (packed && g.nx == 256) xy_fwd_rp_launch<8>(c->stream, g.nz, xa, y1, y2, c->tw[1]);
+  else if (packed && g.nx == 128) xy_fwd_rp_launch<4>(c->stream, g.nz, xa, y1, y2, c->tw[1]);
+  else if (packed) xy_fwd_rp_launch<2>(c->stream, g.nz, xa, y1, y2, c->tw[1]);
   else { TPX_FOUR_STEP_SWITCH(g.nx, L_XYF) }
 #undef L_XYF
   TPX_LAUNCH_CHECK();
