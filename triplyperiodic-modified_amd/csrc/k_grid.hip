@@ -261,11 +261,14 @@ struct ProjArgs {
   double *partials;
   long npart;
   double *scal = nullptr;    // non-null: P0_int = P0_new too (grid.cpp:898)
-  int32_t *zero = nullptr;   // non-null: cleared from zero[1] on, one value a cell
+  int32_t *zero = nullptr;   // non-null: cleared from zero[1] on, one value a cell, and tot
+  int32_t *tot = nullptr;    // totals of the scan blocks of those values
+  int ntot = 0;
   double c_np1, c_new;
   __device__ void to_global() {
     scal = gptr(scal);
     zero = gptr(zero);
+    tot = gptr(tot);
     P = gptr(P);
     for (int q = 0; q < 3; ++q) np1[q] = gptr(np1[q]);
     for (int q = 0; q < 3; ++q) nw[q] = gptr(nw[q]);
@@ -287,7 +290,10 @@ struct k_project {
   double s[3] = {0, 0, 0};
   if (a.scal && blockIdx.x == 0 && threadIdx.x == 0) a.scal[SC_P0_INT] = a.scal[SC_P0_NEW];
   if (ok) {
-    if (a.zero) a.zero[c + 1] = 0;
+    if (a.zero) {
+      a.zero[c + 1] = 0;
+      if (c < a.ntot) a.tot[c << kTotShift] = 0;
+    }
     const double *__restrict__ P = a.P;
     double pc = P[c];
     double gr[3] = {(pc - P[ix(i - 1, j, k)]) * g.idx, (pc - P[ix(i, j - 1, k)]) * g.idy,
@@ -607,6 +613,8 @@ void launch_project(tpx_ctx *c, const Coef &k, const double *P, double *const ru
   ProjArgs a{};
   a.scal = advance_p0 ? c->scal : nullptr;
   a.zero = zero;
+  a.tot = c->tile_tot;
+  a.ntot = scan_blocks(c->g.n);
   a.P = P;
   for (int d = 0; d < 3; ++d) { a.np1[d] = ru_np1[d]; a.nw[d] = ru_new[d]; }
   a.partials = c->partials;

@@ -71,6 +71,8 @@ struct AdvArgs {
   long cstride;
   const int32_t *inv_int;    // particle -> sorted position of x_int
   int32_t *cnt;              // per-cell counts of x_new (start_new + 1) (null: no binning this substep)
+  int32_t *tot;              // with cnt: the scan blocks' totals, block = cell >> tot_shift
+  int tot_shift;
   int32_t *key;
   long n;
   int int_is_base, np1_is_base;  // the int / np1 inputs are the base arrays
@@ -95,6 +97,7 @@ struct AdvArgs {
     contrib = gptr(contrib);
     inv_int = gptr(inv_int);
     cnt = gptr(cnt);
+    tot = gptr(tot);
     key = gptr(key);
   }
 };
@@ -208,7 +211,10 @@ struct k_advance {
   int ki = (int)(nv[0] * g.idx), kj = (int)(nv[1] * g.idy), kz = (int)(nv[2] * g.idz);
   long nk = ix(ki, kj, kz);
   a.key[p] = (int32_t)nk;
-  if (a.cnt) count_runs(a.cnt, (int)nk);  // only lanes past n left early: the active lanes are a prefix
+  if (a.cnt) {  // only lanes past n left early: the active lanes are a prefix
+    count_runs(a.cnt, (int)nk);
+    count_runs(a.tot, (int)nk >> a.tot_shift << kTotShift);
+  }
 }
 };
 
@@ -226,11 +232,13 @@ struct k_keys {
 }
 };
 
-struct k_set_i {
+// cnt = 0; with tot, the scan blocks' totals too
+struct k_zero_counts {
   static constexpr int kBounds = 1024;
-  static __device__ __forceinline__ void run(int32_t *a, int32_t v, long n) {
+  static __device__ __forceinline__ void run(int32_t *cnt, long n, int32_t *tot, int ntot) {
   long p = (long)blockIdx.x * block_dim_x() + threadIdx.x;
-  if (p < n) a[p] = v;
+  if (p < n) cnt[p] = 0;
+  if (tot && p < ntot) tot[p << kTotShift] = 0;
 }
 };
 
@@ -324,10 +332,17 @@ struct k_iota {
 // ---- exclusive scan of int32, in place, in two launches ----
 // A block takes `tiles` consecutive tiles of 4096 values: the first launch
 // leaves each block's total, the second adds up the totals before its own and
-// scans.  Three passes over the values (read; read and write) in place of the
-// six of a scan per block, a scan of the totals, an add per block and a copy
-// for the placement cursors: 131 -> 43 us for the 1.7e7 cells of 64 boxes of
-// 64^3, four launches -> two for a single box.
+// scans.  Where the particle advance counts, it adds to the blocks' totals too
+// and the first launch is left out (plain substeps at 32^3 92 -> 83 us, 64^3
+// 107 -> 104, 128^3 425 -> 418): one atomic per run of particles of one block
+// among a wave's, nearly always one a wave, on a cache line of its own for each
+// total (side by side they queue: 7.9 -> 19.9 us an advance at 64^3, 83 -> 101
+// at 128^3; a line apart 8.3 and 84.6).  The second launch takes its blocks in
+// the order of the placement after it, which then finds its slots in the L2 of
+// its XCD (16.0 -> 11.0 us at 128^3).  Three passes over the values (read;
+// read and write) in place of the six of a scan per block, a scan of the totals,
+// an add per block and a copy for the placement cursors: 131 -> 43 us for the
+// 1.7e7 cells of 64 boxes of 64^3, four launches -> two for a single box.
 constexpr int kScanPer = 16;
 constexpr int kScanTile = kBlock * kScanPer;
 
@@ -365,13 +380,15 @@ struct k_scan_totals {
 
 struct k_scan_apply {
   static constexpr int kBounds = kBlock;
-  static __device__ __forceinline__ void run(int32_t *data, long n, int tiles, const int32_t *__restrict__ totals) {
+  static __device__ __forceinline__ void run(int32_t *data, long n, int tiles, const int32_t *__restrict__ totals,
+                                             int stride_shift) {
     __shared__ int32_t sh[4], st[kScanTile + kScanTile / kScanPer];  // one spare slot every 16: no bank conflicts
     const int tid = (int)threadIdx.x;
+    const unsigned blk = xcd_block(blockIdx.x, gridDim.x);  // as the placement that follows: its slots are in this XCD's L2
     int32_t before = 0;
-    for (unsigned b = threadIdx.x; b < blockIdx.x; b += kBlock) before += totals[b];
+    for (unsigned b = threadIdx.x; b < blk; b += kBlock) before += totals[b << stride_shift];
     before = block_total(before, sh);
-    const long lo = (long)blockIdx.x * tiles * kScanTile;
+    const long lo = (long)blk * tiles * kScanTile;
     for (int t = 0; t < tiles; ++t) {
       const long base = lo + (long)t * kScanTile;
       int32_t v[kScanPer];
@@ -891,14 +908,30 @@ void launch_iota(tpx_ctx *c, int32_t *p, int64_t n) {
   TPX_LAUNCH_CHECK();
 }
 
-void launch_exclusive_scan(tpx_ctx *c, int32_t *data, int64_t n) {
-  // at most 8192 blocks: each reads the totals of all before it
-  int tiles = 1;
-  while ((n + (int64_t)tiles * kScanTile - 1) / ((int64_t)tiles * kScanTile) > 8192) tiles *= 2;
-  const unsigned nb = (unsigned)((n + (int64_t)tiles * kScanTile - 1) / ((int64_t)tiles * kScanTile));
-  tpx_launch<k_scan_totals>(nb, kBlock, 0, c->stream, (const int32_t *)data, (long)n, tiles, c->scan_tmp);
-  TPX_LAUNCH_CHECK();
-  tpx_launch<k_scan_apply>(nb, kBlock, 0, c->stream, data, (long)n, tiles, (const int32_t *)c->scan_tmp);
+// scan blocks of n values: at most 8192, each reads the totals of all before it
+static int scan_shift(int64_t n) {
+  int shift = 12;
+  static_assert(kScanTile == 1 << 12, "a scan tile is 2^12 values");
+  while ((n + (1LL << shift) - 1) >> shift > 8192) ++shift;
+  return shift;
+}
+
+int scan_blocks(int64_t n) {
+  const int shift = scan_shift(n);
+  return (int)((n + (1LL << shift) - 1) >> shift);
+}
+
+// totals: the blocks' totals where they are known (null: a launch of their own)
+static void launch_exclusive_scan(tpx_ctx *c, int32_t *data, int64_t n, const int32_t *totals) {
+  const int tiles = 1 << (scan_shift(n) - 12);
+  const unsigned nb = (unsigned)scan_blocks(n);
+  const int stride_shift = totals ? kTotShift : 0;
+  if (!totals) {
+    tpx_launch<k_scan_totals>(nb, kBlock, 0, c->stream, (const int32_t *)data, (long)n, tiles, c->scan_tmp);
+    TPX_LAUNCH_CHECK();
+    totals = c->scan_tmp;
+  }
+  tpx_launch<k_scan_apply>(nb, kBlock, 0, c->stream, data, (long)n, tiles, totals, stride_shift);
   TPX_LAUNCH_CHECK();
 }
 
@@ -908,17 +941,19 @@ void launch_exclusive_scan(tpx_ctx *c, int32_t *data, int64_t n) {
 // leaves each cell's first slot at start[c + 1], the placement moves it on to
 // one past its last, which is the first slot of cell c + 1: start is then the
 // CSR, with no cursors of its own.
-static void bin_particles(tpx_ctx *c, const int32_t *key, int32_t *perm, int32_t *inv, int32_t *start) {
+static void bin_particles(tpx_ctx *c, const int32_t *key, int32_t *perm, int32_t *inv, int32_t *start,
+                          const int32_t *totals = nullptr) {
   Particles &pt = c->pt;
   long n = pt.n, nc = c->g.n;
-  launch_exclusive_scan(c, start + 1, nc);
+  launch_exclusive_scan(c, start + 1, nc, totals);
   tpx_launch<k_place>(grid1d(n, kBlock), kBlock, 0, c->stream, key, start + 1, perm, n);
   tpx_launch<k_fixup>(grid1d(nc, kBlock), kBlock, 0, c->stream, start, perm, inv, nc);
   TPX_LAUNCH_CHECK();
 }
 
-static void zero_counts(tpx_ctx *c, int32_t *cnt) {
-  tpx_launch<k_set_i>(grid1d(c->g.n + 1, kBlock), kBlock, 0, c->stream, cnt, 0, c->g.n + 1);
+static void zero_counts(tpx_ctx *c, int32_t *cnt, int32_t *tot = nullptr) {
+  tpx_launch<k_zero_counts>(grid1d(c->g.n + 1, kBlock), kBlock, 0, c->stream, cnt, (long)c->g.n + 1, tot,
+                            scan_blocks(c->g.n));
   TPX_LAUNCH_CHECK();
 }
 
@@ -953,6 +988,8 @@ void launch_particle_advance(tpx_ctx *c, const Coef &k, const double *const ru_i
   a.cstride = pt.cap;
   a.inv_int = pt.inv_int;
   a.cnt = count_new ? pt.start_new + 1 : nullptr;
+  a.tot = c->tile_tot;
+  a.tot_shift = scan_shift(c->g.n);
   a.key = pt.key;
   a.n = pt.n;
   a.int_is_base = pt.int_is_base || si == sb;
@@ -969,7 +1006,7 @@ void launch_particle_advance(tpx_ctx *c, const Coef &k, const double *const ru_i
   a.rk3 = k.rk == 3;
   if (count_new) {
     timing_begin(c, TPX_K_SORT);
-    if (!pt.new_zeroed) zero_counts(c, pt.start_new);
+    if (!pt.new_zeroed) zero_counts(c, pt.start_new, c->tile_tot);
     pt.new_zeroed = false;
     timing_end(c, TPX_K_SORT);
   }
@@ -1121,7 +1158,7 @@ void launch_sort_new(tpx_ctx *c) {
   if (pt.n == 0) return;
   if (!pt.new_counted) throw std::logic_error("x_new was not counted by the particle advance");
   timing_begin(c, TPX_K_SORT);
-  bin_particles(c, pt.key, pt.perm_new, pt.inv_new, pt.start_new);
+  bin_particles(c, pt.key, pt.perm_new, pt.inv_new, pt.start_new, c->tile_tot);
   timing_end(c, TPX_K_SORT);
   pt.new_counted = false;
 }

@@ -893,7 +893,8 @@ int tpx_create(const tpx_params *p, int64_t np_capacity, tpx_ctx **out) {
     // one partial per 256-cell block or per x-row, whichever is more
     c->n_partials = std::max((long)grid1d(g.n, 256), (long)g.ny * g.nz) + 1024;
     dalloc(&c->partials, 3 * (size_t)c->n_partials);
-    ialloc(&c->scan_tmp, 8192);  // block totals of a scan
+    ialloc(&c->scan_tmp, 8192 + ((size_t)scan_blocks(g.n) << kTotShift));  // block totals of a scan, and those the advance counts
+    c->tile_tot = c->scan_tmp + 8192;
     // one pinned block (each allocation costs some 0.3 ms here and as much
     // again to free): the scalars' mirror, the solves' loop state on a line of
     // its own, and the first copying thread's chunks

@@ -104,7 +104,7 @@ struct Particles {
   int32_t *inv_int = nullptr, *inv_new = nullptr;       // particle -> sorted position
   int32_t *start_int = nullptr, *start_new = nullptr;   // CSR over cells (n_cell+1)
   bool new_counted = false;       // the last advance counted x_new into start_new
-  bool new_zeroed = false;        // start_new is all zero: the next advance can count into it
+  bool new_zeroed = false;        // start_new and tile_tot are all zero: the next advance can count into them
   bool has_tau = false, has_eps = false;
   // spare arrays the step-end permutation writes into (rhs_t, tau, eps, flag)
   double *spare[3] = {};
@@ -347,6 +347,7 @@ struct tpx_ctx {
   long n_partials = 0;
   double *h_scal = nullptr;       // pinned host mirror of scal
   int32_t *scan_tmp = nullptr;    // scan block totals
+  int32_t *tile_tot = nullptr;    // those of the counts of x_new (beside scan_tmp; zero whenever pt.new_zeroed)
   tpx::Particles pt;
   tpx::Timing tm;
   tpx::HostStage stage;
@@ -438,7 +439,8 @@ void launch_iota(tpx_ctx *c, int32_t *p, int64_t n);
 // inv its inverse.  launch_zero_counts clears the cells + 1 counts.
 void launch_bin_by_key(tpx_ctx *c, const int32_t *key, int32_t *perm, int32_t *inv, int32_t *start);
 void launch_zero_counts(tpx_ctx *c, int32_t *cnt);
-void launch_exclusive_scan(tpx_ctx *c, int32_t *data, int64_t n);  // in place
+constexpr int kTotShift = 5;  // totals counted by atomics lie a cache line apart
+int scan_blocks(int64_t n);  // blocks of a scan of n values, and their totals
 
 // memory of the adjoint's arrays (tpx_api.hip): null when the device is full
 void *tape_alloc(AdjointTape &t, size_t bytes);
