@@ -472,11 +472,15 @@ void launch_rhs_ru(tpx_ctx *c, const Coef &k, bool with_rho, const double *const
   // batch) has fewer than 1024 blocks, down to 2.  Each block re-reads two
   // halo planes of the four raw fields, so a short march costs bandwidth, but
   // a small launch needs the blocks: one 64^3 box runs 128 -> 20 us at 2
-  // planes, one 128^3 box 170 -> 84 us at 8; 64 boxes of 64^3 keep 32.
+  // planes, one 128^3 box 170 -> 84 us at 8; 64 boxes of 64^3 keep 32.  Where
+  // two planes leave fewer than 256 blocks, one a CU, single planes: 32^3
+  // 13.5 -> 9.8 us (at 64^3, with 512 blocks at two planes, single planes are
+  // slower, 17.9 -> 19.7).
   zg.KC = g.nz < 32 ? g.nz : 32;
   {
     const long cols = (long)(g.nx / zg.TX) * (g.ny / zg.TY) * (g_rec ? g_rec->nbox : 1u);
     while (zg.KC > 2 && zg.KC % 2 == 0 && cols * (g.nz / zg.KC) < 1024) zg.KC /= 2;
+    if (zg.KC == 2 && cols * (g.nz / zg.KC) < 256) zg.KC = 1;
   }
   unsigned nb = (unsigned)((g.nx / zg.TX) * (g.ny / zg.TY) * (g.nz / zg.KC));
   int threads = zg.TX * zg.TY;
