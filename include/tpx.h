@@ -160,11 +160,13 @@ int tpx_poisson_solve(tpx_ctx *ctx, const double *cx, const double *cy, const do
  * guess and overwritten), allocating nothing.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * The residual it iterates on lives in a file-scope static device array of
- * 2^21 doubles (16 MiB) per GPU, held until the process ends, so grids of
- * more than 2^21 cells (128^3) are rejected with TPX_E_ARG.  Every call on one
- * GPU shares that GPU's array: calls that overlap on one GPU (two contexts on
- * two host threads) race.  The call returns when the solve has ended. */
+ * Grids of more than 2^21 cells (128^3) are rejected with TPX_E_ARG: the
+ * residual, where it is not formed inside the first transform pass (an axis
+ * length of 8, y and z lengths both 512, or x length 512 with arrays that are
+ * not 16-byte aligned), lives in a file-scope static device array of 2^21
+ * doubles (16 MiB) per GPU, held until the process ends.  Calls of that form
+ * share the GPU's array: two that overlap on one GPU (two contexts on two host
+ * threads) race.  The call returns when the solve has ended. */
 int tpx_poisson_solve_device(tpx_ctx *ctx, const double *cx, const double *cy, const double *cz, double *P,
                              const double *rhs, int *iterations);
 int tpx_time_advance_rk4(tpx_ctx *ctx);              /* grid.cpp:890-900 */

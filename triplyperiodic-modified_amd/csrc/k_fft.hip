@@ -1995,11 +1995,11 @@ unsigned three_pass_launch(tpx_ctx *c, const XArgs &xa, const XInvArgs &xi, cons
   const int mxh = g.nx / 2 + 1;
   const unsigned nb13 = (unsigned)(g.nz * y1);
   const size_t sh13 = std::max(sizeof(double) * (size_t)y2 * r2 * (r1 + 1), sizeof(double2) * (size_t)mxh * (y2 + 1));
-  // pass 1 at x lengths 64, 128 and 256 takes the packed real-row transform
-  // unless TPX_XPACK=0 asks for the full-length complex one; pass 3 keeps
-  // the full-length inverse (the same half spectrum either way: the packed
-  // inverse, whose final stage leaves half the block idle over the P
-  // update, measured slower)
+  // pass 1 at x lengths 64, 128, 256 and 512 takes the packed real-row transform
+  // unless TPX_XPACK=0 asks for the full-length complex one (512 has no other
+  // here: it then takes the five passes); pass 3 keeps the full-length inverse
+  // below 512 (the same half spectrum either way: the packed inverse, whose
+  // final stage leaves half the block idle over the P update, measured slower)
   // the packed form reads pairs with 16-byte loads: the library's own fields
   // are aligned, a caller's arrays (coefficient solve) need not be
   bool packed = (g.nx == 64 || g.nx == 128 || g.nx == 256 || g.nx == 512) && c->x_packed;
