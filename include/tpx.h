@@ -166,7 +166,8 @@ int tpx_poisson_solve(tpx_ctx *ctx, const double *cx, const double *cy, const do
  * not 16-byte aligned), lives in a file-scope static device array of 2^21
  * doubles (16 MiB) per GPU, held until the process ends.  Calls of that form
  * share the GPU's array: two that overlap on one GPU (two contexts on two host
- * threads) race.  The call returns when the solve has ended. */
+ * threads) race.  The call returns when the solve has ended and nothing it
+ * queued reads or writes the arrays any more, with an error code as without. */
 int tpx_poisson_solve_device(tpx_ctx *ctx, const double *cx, const double *cy, const double *cz, double *P,
                              const double *rhs, int *iterations);
 int tpx_time_advance_rk4(tpx_ctx *ctx);              /* grid.cpp:890-900 */
