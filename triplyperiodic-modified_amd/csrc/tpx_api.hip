@@ -451,13 +451,17 @@ int wait_iterations(tpx_ctx *c, int want, bool &stopped) {
 // queues `guess` iterations, and while the solve has not stopped then, two
 // more and one for each that ends.  Returns the iterations that ran.
 //
-// `drain`: the iterations read arrays that are the caller's again on return.
-// Where more iterations were queued than ran, the host heard of the stop from
-// the pass 1 that was one too many, whose other blocks may still be reading, so
-// the stream is waited for; where all of them ran it heard from the loop check
-// behind the last, and nothing that reads is left.  (A wait after every solve
-// costs 40 us: 225 against 190 us for the 12 iterations at 32^3.)
-int solve_loop(tpx_ctx *c, int guess, const std::function<void(int)> &iterate, bool drain = false) {
+// `callers`: a solve of the caller's system.  Its counts may jump from call to
+// call, so only four of the guess are queued ahead of those that ended (all at
+// once, a solve of one iteration at 32^3 after one of 12 took 130-175 us for 90, and
+// 140-184 for 98 at 128^3; the step's solves, whose counts change slowly, gain
+// nothing by it).  And its arrays are the caller's again on return: where more
+// iterations were queued than ran, the host heard of the stop from the pass 1
+// that was one too many, whose other blocks may still be reading, so the stream
+// is waited for; where all of them ran it heard from the loop check behind the
+// last, and nothing that reads is left.  (A wait after every solve costs 40 us:
+// 225 against 190 us for the 12 iterations at 32^3.)
+int solve_loop(tpx_ctx *c, int guess, const std::function<void(int)> &iterate, bool callers = false) {
   if (!(0 < c->Iteration && 100.0 > c->p.epsilon)) {  // err = 100 before the first (poisson.cpp:391-396)
     launch_solve_begin(c);
     return 0;
@@ -469,24 +473,29 @@ int solve_loop(tpx_ctx *c, int guess, const std::function<void(int)> &iterate, b
     }
     ~Running() { c->iter_ctl = {}; }
   } running(c);
-  int queued = 0;
+  const int expected = std::min(std::max(1, guess), c->Iteration), ahead = callers ? 4 : expected;
+  int queued = 0, its = 0;
+  bool stopped = false;
   auto queue = [&](int n) {
     for (; n > 0 && queued < c->Iteration; --n) {
       iterate(queued++);
       c->iter_ctl.first = 0;
       ++c->iter_ctl.index;
     }
-    launch_loop_check(c);
+    if (queued >= expected) launch_loop_check(c);
   };
-  queue(std::max(1, guess));
-  bool stopped = false;
-  int its = wait_iterations(c, queued, stopped);
+  queue(std::min(expected, ahead));
+  while (!stopped && queued < expected) {
+    its = wait_iterations(c, queued - (ahead - 1), stopped);
+    if (!stopped) queue(1);
+  }
+  if (!stopped) its = wait_iterations(c, queued, stopped);
   if (!stopped) queue(1);
   while (!stopped) {  // the iteration count stops it at the latest
     queue(1);
     its = wait_iterations(c, std::max(its + 1, queued - 1), stopped);
   }
-  if (drain && its < queued) sync(c);
+  if (callers && its < queued) sync(c);
   return its;
 }
 
@@ -502,10 +511,9 @@ void do_solve_poisson(tpx_ctx *c, int rk, int *iters, const std::function<void(i
 }
 
 // poisson::FFT with the caller's face coefficient (poisson.cpp:391-411).  P,
-// RHS, C and res (work) are dense device arrays; drain as in solve_loop.
-void do_solve_coef(tpx_ctx *c, const double *const cf[3], double *P, const double *rhs, double *res, int *iters,
-                   bool drain = false) {
-  const int i = solve_loop(c, c->coef_guess, [&](int) { launch_coef_iteration(c, cf, P, rhs, res); }, drain);
+// RHS, C and res (work) are dense device arrays.
+void do_solve_coef(tpx_ctx *c, const double *const cf[3], double *P, const double *rhs, double *res, int *iters) {
+  const int i = solve_loop(c, c->coef_guess, [&](int) { launch_coef_iteration(c, cf, P, rhs, res); }, true);
   c->coef_guess = i;
   c->num_iteration = i;  // the reference's poisson object keeps the last solve's count
   if (iters) *iters = i;
@@ -1327,7 +1335,7 @@ int tpx_poisson_solve_device(tpx_ctx *ctx, const double *cx, const double *cy, c
     if (!ctx->static_scratch) throw std::logic_error("static scratch not set up");
     const double *cf[3] = {cx, cy, cz};
     try {
-      do_solve_coef(ctx, cf, P, rhs, ctx->static_scratch, iterations, true);
+      do_solve_coef(ctx, cf, P, rhs, ctx->static_scratch, iterations);
     } catch (...) {  // what is queued reads the caller's arrays
       (void)hipStreamSynchronize(ctx->stream);
       throw;
