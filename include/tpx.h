@@ -232,7 +232,11 @@ int tpx_ensemble_step(tpx_ctx *const *ctxs, int n, int nsteps, int concurrency);
  * first RHS_T is taken as the exchange of its initial state, as
  * tpx_initialize and every step's end form it.  Any output may be null.
  * tpx_adjoint_release frees the tape (nsteps x 20 grid fields, + 12 under
- * two-way coupling, + 4 with the heat exchange) and the sweep's work arrays. */
+ * two-way coupling, + 4 with the heat exchange) and the sweep's work arrays.
+ * Until then the context keeps that memory: the next recording of the same
+ * length, interval, particle count and options takes it over; any other one
+ * gives it back first if it is more than 1 GiB.  What two recordings had no
+ * use for is given back too, and all that is unused when the device is full. */
 int tpx_adjoint_record(tpx_ctx *ctx, int nsteps, int every, double *J);
 int tpx_adjoint_gradient(tpx_ctx *ctx, double *dJ_dtau, double *dJ_dstate);
 int tpx_adjoint_gradient_full(tpx_ctx *ctx, double *dJ_dtau, double *dJ_dstate, double *dJ_dA, double *dJ_dRU,

@@ -700,8 +700,6 @@ void step_end(tpx_ctx *c) {
   do_time_advance(c, true);
 }
 
-// The arrays of a recorded adjoint run go back to the tape's blocks
-// (adjoint_free), which the next recording's take.
 // Gives the unused blocks of a tape back to the device (min_idle: those unused
 // over so many recordings)
 void tape_give_back(AdjointTape &t, int min_idle) {
@@ -713,6 +711,8 @@ void tape_give_back(AdjointTape &t, int min_idle) {
   t.blocks.resize(m);
 }
 
+// The arrays of a recorded adjoint run go back to the tape's blocks, which the
+// next recording's take.
 void adjoint_free(AdjointTape &t) {
   auto f = [](auto *&p) { p = nullptr; };
   f(t.gas); f(t.ckpt); f(t.y); f(t.seg); f(t.lb); f(t.lnext); f(t.S); f(t.stage); f(t.lam); f(t.dtau); f(t.djdc);
@@ -2132,6 +2132,15 @@ int tpx_adjoint_record(tpx_ctx *ctx, int nsteps, int every, double *J) {
     t.heat = heat_active(c);
     t.nq = t.heat ? 7 : 6;
     const long n = c->g.n, np = pt.n;
+    // a recording of the last one's shape takes all its blocks again; one of
+    // another shape would hold both, which only small tapes may
+    const std::array<long, 8> shape{nsteps, every, np, t.mode, t.heat, c->p.twc != 0, pt.has_tau, pt.has_eps};
+    if (shape != t.shape) {
+      size_t kept = 0;
+      for (const AdjointTape::Block &b : t.blocks) kept += b.bytes;
+      if (kept > AdjointTape::kTapeKept) tape_give_back(t, 0);
+      t.shape = shape;
+    }
     const size_t nq = (size_t)t.nq;
     auto alloc = [&](auto **p, size_t count) {
       *p = static_cast<std::remove_reference_t<decltype(**p)> *>(tape_alloc(t, sizeof(**p) * count));

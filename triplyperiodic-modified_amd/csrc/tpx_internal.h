@@ -13,6 +13,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <array>
 #include <functional>
 #include <stdexcept>
 #include <string>
@@ -209,9 +210,12 @@ struct AdjointTape {
   GasAdjoint ga{};
   // device memory of the arrays above, kept from one recording to the next (a
   // recording's allocations and frees took longer than its steps) and given
-  // back on release, when the device is full, or unused over two recordings
+  // back on release, when the device is full, unused over two recordings, or,
+  // above kTapeKept, before a recording of another shape
   struct Block { void *p; size_t bytes; bool used; int idle; };
   std::vector<Block> blocks;
+  static constexpr size_t kTapeKept = 1u << 30;
+  std::array<long, 8> shape{};  // steps, checkpoint interval, particles, tape mode and switches of the recording
   // steps the gas and sub tapes hold
   int tape_steps() const { return segmented ? std::min(every, nsteps) : nsteps; }
   // the gas tape of step s (4 substeps x 4 fields of n)
