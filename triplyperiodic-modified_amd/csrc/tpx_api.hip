@@ -13,10 +13,10 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
+#include "host_team.h"
 #include "tpx_internal.h"
 
 using namespace tpx;
@@ -300,13 +300,7 @@ void transfer(tpx_ctx *c, const HostPart *part, int nparts, bool up) {
     drain(1);
     if (e != hipSuccess) failed = (int)e;
   };
-  std::vector<std::thread> helpers;
-  try {
-    for (int t = 1; t < threads; ++t) helpers.emplace_back(work, t);
-  } catch (const std::system_error &) {  // no more threads: the ones that started take all pieces
-  }
-  work(0);
-  for (auto &h : helpers) h.join();
+  run_team(threads, work);
   hip_check((hipError_t)failed.load(), what);
 }
 
