@@ -685,7 +685,7 @@ struct RegDft<16, INV> {
 // e^{-2 pi i k/32}, k < 16
 __device__ __forceinline__ double2 w32(int k) {
   constexpr double c[9] = {1.0, 0.9807852804032304, 0.9238795325112867, 0.8314696123025452, 0.7071067811865476,
-                           0.5555702330196022, 0.3826834323650898, 0.1950903220161283, 0.0};  // cos(pi q/16)
+                           0.5555702330196022, 0.3826834323650898, 0.19509032201612828, 0.0};  // cos(pi q/16)
   return k <= 8 ? make_double2(c[k], -c[8 - k]) : make_double2(-c[16 - k], -c[k - 8]);
 }
 
