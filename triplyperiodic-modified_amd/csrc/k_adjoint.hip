@@ -273,8 +273,7 @@ struct k_adj_gather_pull {
   }
 };
 
-// Keys and counts of the bins of positions (x, y, z rows of Y): the gather's
-// cell (floor), or with cic set the cloud-in-cell base corner (round - 1)
+// out = (a + b) + d, and out[q] = src[idx[q]]: the sweep's outputs
 struct k_sum3 {
   static constexpr int kBounds = kBlock;
   static __device__ __forceinline__ void run(const double *__restrict__ a, const double *__restrict__ b,
@@ -293,6 +292,8 @@ struct k_take {
   }
 };
 
+// Keys and counts of the bins of positions (x, y, z rows of Y): the gather's
+// cell (floor), or with cic set the cloud-in-cell base corner (round - 1)
 struct k_adj_bin_keys {
   static constexpr int kBounds = kBlock;
   static __device__ __forceinline__ void run(const Geo &g, const double *Y, int cic, int32_t *key, int32_t *cnt,
@@ -708,7 +709,6 @@ StepArgs step_args(tpx_ctx *c, int step, const double *const yin[7], double *con
 
 }  // namespace
 
-// copies this substep's RU_int and Rho_int into the tape
 void launch_sum3(tpx_ctx *c, const double *a, const double *b, const double *d, double *out, long n) {
   tpx_launch<k_sum3>(grid1(n), kBlock, 0, c->stream, a, b, d, out, n);
   TPX_LAUNCH_CHECK();
@@ -719,6 +719,7 @@ void launch_take(tpx_ctx *c, const double *src, const int32_t *idx, double *out,
   TPX_LAUNCH_CHECK();
 }
 
+// copies this substep's RU_int and Rho_int into the tape
 void adjoint_tape_substep(tpx_ctx *c, int rk, const double *const ru_int[3], const double *rho_int) {
   AdjointTape &t = c->adj;
   if (t.step < 0) return;

@@ -410,8 +410,9 @@ void do_update_ru_wop(tpx_ctx *c, int rk, bool with_rho, bool with_p0 = false) {
 
 // Waits until the running solve has stopped or finished `want` iterations;
 // returns the iterations finished, and whether it has stopped.  The loop state
-// is read from pinned memory that the device writes after every iteration: the
-// next launch follows a couple of microseconds after the solve ends, where a
+// is read from pinned memory that the device writes after every iteration (the
+// three-pass form from the next iteration's pass 1, or from the loop check
+// behind the last one queued): the next launch follows a couple of microseconds after the solve ends, where a
 // copy of the state and a stream wait, once per two iterations, left the GPU
 // idle (a 12-iteration solve at 32^3 401 -> 250-285 us, 13 at 128^3 906 ->
 // 820-846; 40 steps at 32^3 with two iterations a solve 21.4 -> 16.4 ms).  A
