@@ -1964,9 +1964,9 @@ bool aligned16(std::initializer_list<const void *> p) {
 // y2 / z1, z2: the four-step factors of x, y and z.  An x length of 512 has only
 // the packed rows (16 x 16 points of pairs), which need 16-byte aligned fields:
 // `aligned`.
-// An axis of 512 took the five-pass form with Stockham transforms before; one
-// iteration: 512 x 64 x 128 154 -> 95 us, 64 x 512 x 128 179 -> 124, 64 x 128 x
-// 512 167 -> 116, 128 x 256 x 512 650 -> 469, 512 x 32 x 512 347 -> 205.
+// The five-pass form, which axes of 512 took before, and this one, kernel time
+// an iteration: 512 x 64 x 128 156 and 80 us, 64 x 512 x 128 172 and 100, 64 x
+// 128 x 512 162 and 103, 128 x 256 x 512 635 and 411, 512 x 32 x 512 328 and 187.
 bool three_pass_shape(const tpx_ctx *c, int &r1, int &r2, int &y1, int &y2, int &z1, int &z2, bool aligned = true) {
   const Geo &g = c->g;
   // 512 = 32 x 16 along y (16 rows a block in passes 1 and 3), 16 x 32 along z
